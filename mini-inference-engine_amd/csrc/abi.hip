@@ -41,6 +41,7 @@ int linear_layout(int64_t M, int64_t N, int64_t K, int config, LinearLayout* L) 
   if (st != MI355X_FP8_OK) return st;
   L->kb = cdiv64(K, 128);
   L->kpad = L->kb * 128;
+  L->plan.q_padded = true;  // the quantizer writes zero codes up to kpad
   L->mpad = cdiv64(M > 0 ? M : 1, 64) * 64;
   L->gemm_bytes = gemm_workspace_bytes(L->plan);
   L->q_off = align256(L->gemm_bytes);

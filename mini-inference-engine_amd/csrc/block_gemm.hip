@@ -850,6 +850,8 @@ int64_t device_cus() {
 // rows takes 192 x 160: 1-3 % either way against 256 x 128.)
 // A last, partly filled wave costs 0.7 + 0.3 x its fill of a full one (a half-filled wave
 // measured 0.75-0.98).  Every kernel gives the same bits, so the choice may follow M.
+// (The figures rank the tiles; the 128-row kernel's single waves have since become 10-20 % faster
+// in the same order, and launch_block_gemm shortens its tiles to 96 rows where those fit.)
 namespace {
 struct TileVariant {
   int rows, bn;
@@ -1002,13 +1004,15 @@ int launch_block_gemm(const GemmPlan& plan, const uint8_t* q, int64_t ldq, const
                       int64_t ws_sn, int64_t ws_sk, void* out, int out_dtype, int64_t ldo,
                       int64_t M, int64_t N, int64_t K, void* workspace, hipStream_t stream) {
   if (M == 0 || N == 0) return MI355X_FP8_OK;
-  const bool dma_ok = tile_dma_supported(q, ldq, as_sm, as_sk, w, ldw, M, K);
+  const bool dma_ok = tile_dma_supported(q, ldq, as_sm, as_sk, w, ldw, M, K, plan.q_padded);
+  // The 256-row kernel takes whole K groups only, and a forced variant keeps its own bounds.
+  const bool whole = K % kGroup == 0;
   if (plan.kernel >= MI355X_FP8_CONFIG_DMA128_64) {
     // A forced variant: the LDS-DMA preconditions, and for 256- and 192-row tiles their 32-bit
     // offsets.
     static constexpr int kWidth[] = {64, 128, 160, 128, 160, 192, 224, 256, 128, 160, 192, 224, 256, 64, 128};
     const int bn = kWidth[plan.kernel - MI355X_FP8_CONFIG_DMA128_64];
-    if (!dma_ok) return MI355X_FP8_ERR_UNSUPPORTED;
+    if (!dma_ok || !whole) return MI355X_FP8_ERR_UNSUPPORTED;
     if (plan.kernel <= MI355X_FP8_CONFIG_DMA128_160)
       return launch_tile_dma(q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, out, out_dtype, ldo, M, N, K, bn, 128, stream);
     if (plan.kernel >= MI355X_FP8_CONFIG_DMA64_64)
@@ -1018,12 +1022,19 @@ int launch_block_gemm(const GemmPlan& plan, const uint8_t* q, int64_t ldq, const
                           stream);
   }
   if (plan.kernel == MI355X_FP8_CONFIG_TILE256) {
-    if (!dma_ok) return MI355X_FP8_ERR_UNSUPPORTED;
+    if (!dma_ok || !whole) return MI355X_FP8_ERR_UNSUPPORTED;
     return launch_tile256(q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, out, out_dtype, ldo, M, N, K,
                           tile256_width(M, N, device_cus()), 256, stream);
   }
   if (plan.kernel == MI355X_FP8_CONFIG_TILE128 && dma_ok) {
-    const PrefillChoice c = choose_prefill(M, N, device_cus(), tile256_offsets_ok(ldq, ldw, M, N, K));
+    const int64_t cus = device_cus();
+    PrefillChoice c = choose_prefill(M, N, cus, whole && tile256_offsets_ok(ldq, ldw, M, N, K));
+    // 128-row tiles in 96 rows where those still fit one per CU: more CUs share the rows, and a
+    // tile's serial K loop has a quarter less to multiply and a sixth less to load per step.
+    // Measured 128 against 96 rows (us, weights from HBM, N = 2560): 64 wide, K = 9728 at 512
+    // rows 34.1 / 26.9, at 536 27.9 / 27.6, K = 4096 at 536 12.6 / 12.2; 128 wide, K = 4096 at
+    // 1024 rows 21.3 / 18.4, K = 9728 48.3 / 41.1.
+    if (c.rows == 128 && c.bn <= 128 && cdiv(M, 96) * cdiv(N, c.bn) <= cus) c.rows = 96;
     if (c.rows > 128)
       return launch_tile256(q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, out, out_dtype, ldo, M, N, K, c.bn, c.rows,
                             stream);

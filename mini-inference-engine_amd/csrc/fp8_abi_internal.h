@@ -30,6 +30,7 @@ struct GemmPlan {
   int token_tiles;  // stream kernel: 16-token MFMA tiles per slice (1 or 2)
   int row_tiles;    // stream kernel: 16-row MFMA tiles of W per workgroup (1 to 5)
   int rows;         // stream kernel: W rows per workgroup (at most 16 row_tiles)
+  bool q_padded;    // the activation codes reach 128 ceil(K / 128) columns, zero past K (the linear's own)
 };
 
 int plan_gemm(int64_t M, int64_t N, int64_t K, int config, GemmPlan* plan);
@@ -66,10 +67,11 @@ int launch_norm_gate_up_silu(const uint16_t* x, int64_t sxm, const uint16_t* res
                              const float* ws, int64_t ws_sn, int64_t ws_sk, uint16_t* h, int64_t ldh, int64_t M,
                              int64_t N, int64_t K, hipStream_t stream);
 
-// LDS-DMA pipelined prefill kernel (tile_gemm_dma.hip) and its preconditions.
+// LDS-DMA pipelined prefill kernel (tile_gemm_dma.hip) and its preconditions.  With q_padded (the
+// activation codes are zero up to a whole group past K) K may be any multiple of 16.
 bool tile_dma_supported(const uint8_t* q, int64_t ldq, int64_t as_sm, int64_t as_sk, const uint8_t* w,
-                        int64_t ldw, int64_t M, int64_t K);
-// bn: tile width, 64, 128 or 160; rows: tile rows, 128, or 64 (widths 64 and 128).
+                        int64_t ldw, int64_t M, int64_t K, bool q_padded);
+// bn: tile width, 64, 128 or 160; rows: tile rows, 128, or 96 or 64 (widths 64 and 128).
 int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_sk, const uint8_t* w,
                     int64_t ldw, const float* ws, int64_t ws_sn, int64_t ws_sk, void* out, int out_dtype,
                     int64_t ldo, int64_t M, int64_t N, int64_t K, int bn, int rows, hipStream_t stream);

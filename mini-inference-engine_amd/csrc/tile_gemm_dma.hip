@@ -3,31 +3,44 @@
 // Same arithmetic and lane layout as tile_gemm_kernel (block_gemm.hip): one
 // v_mfma_f32_16x16x128_f8f6f4 per 128-wide K group and 16x16 output tile, folded into the
 // fp32 accumulator as acc = fma(partial, a_s * w_s, acc); 128 x BN output tile per
-// 256-thread workgroup (BN = 64, 128 or 160), 2x2 waves of 64 x BN/2.  BN = 160 gives the
+// 256-thread workgroup (BN = 64, 128 or 160), 2x2 waves of 64 x BN/2, and the same with 96 or
+// 64 rows (BN = 64 or 128).  BN = 160 gives the
 // Qwen3-4B o_proj and down projections at M = 2048 exactly 256 tiles (16 x 16) instead
 // of 320; a wave's columns may then straddle two 128-column weight-scale blocks, so each
 // 16-column MFMA tile uses its own block's scale.
 //
 // What differs is the feed: global memory goes straight into LDS with
 // global_load_lds_dwordx4 (no register staging, no ds_write), through a ring of STAGES
-// stages (2 when two workgroups share a CU; when the tiles do not fill the CUs, 3, or 4 for
-// BN = 64).  Each stage holds the W tile (BN rows x 128 B), the activation tile
+// stages (2 when two workgroups share a CU, else 4).  Each stage holds the W tile (BN rows x 128 B), the activation tile
 // (128 x 128 B) and the 128 activation scales of its K group.  A 64-lane DMA instruction fills 1 KiB of LDS
 // linearly (lane i -> byte 16 i), i.e. 8 rows of 8 16-byte chunks; the XOR swizzle
 // (physical chunk p of row r holds logical chunk p ^ (r & 7)) is applied by choosing each
 // lane's source address, so the MFMA fragment reads (ds_read_b128) are bank-conflict free.
 //
-// With one wave per SIMD nothing else hides a wave's LDS reads, so each K step is
-// software-pipelined (k_step): the fragments its first MFMAs need are read during the
-// previous step, each later weight fragment is read while the MFMAs of the one before run,
-// and the workgroup barrier sits between the two parts of a step rather than in front of
-// it.  The K loop is unrolled by STAGES so that every stage index is a compile-time
+// One workgroup per CU (four stages, one wave per SIMD): nothing else hides a wave's LDS reads,
+// so the fragments of a K group are read into registers one whole step before its MFMAs, while
+// the previous group's run (reg_step; a wave has 512 registers).  A step then costs the larger
+// of its feed and its MFMAs plus one barrier.  What bounds it is the feed: for 128x64 tiles over
+// K = 9728 at 536 rows a step takes 0.33 us, 0.24 us without the DMA and 0.11 us of MFMA; more
+// stages, no barrier and no fold each change it by less than 4 %.  Measured against the former
+// step, which read the fragments of its first MFMAs during the previous step only (us, weights
+// from HBM): N = 2560 at 536 rows K = 4096 17.1 -> 14.3, K = 9728 32.6 -> 28.0; at 2048 rows
+// (128x160) 59.1 -> 57.9.
+// Two workgroups per CU (two stages, k_step; also 256 registers at most): the two hide each
+// other's waits; a K step reads the fragments of its first MFMAs during the previous step, each
+// later weight fragment while the MFMAs of the one before run, and the barrier sits between the
+// two parts.  The K loop is unrolled by STAGES so that every stage index is a compile-time
 // constant.
+//
+// K need not be whole groups when the activation codes are padded with zeros to one (the
+// linear's own codes): the weight chunks past K then read other codes of the same row, times zero
+// (KTAIL).  An fp16 linear of 333 x 2880 x 2880 went from 33.1 us on the register-staged kernel
+// to 16.8 us.
 //
 // The output tile leaves through LDS as full-row 16-byte non-temporal stores when the output
 // rows are 16-byte aligned (staged_index, fp8_common.h), else straight from the registers.
 //
-// Preconditions (checked by the launcher): K % 128 == 0, W/q base pointers and leading
+// Preconditions (checked by the launcher): K % 128 == 0 (% 16 with padded codes), W/q base pointers and leading
 // dimensions 16-byte aligned, activation scales K-group-major (as_sm == 1) with row
 // length as_sk >= M, row strides below 2^32 / 159 bytes (W) and 2^32 / 127 bytes (q), so that
 // the 32-bit per-lane offsets within a tile reach every row.  Out-of-range tile rows read the
@@ -39,15 +52,8 @@ namespace mi355x {
 namespace {
 
 constexpr int kDmaThreads = 256;
-#ifndef MI355X_DMA_STAGES_FEW
-#define MI355X_DMA_STAGES_FEW 3  // ring depth when the tiles do not exceed the CUs
-#endif
-#ifndef MI355X_DMA_STAGES_FEW_NARROW
-#define MI355X_DMA_STAGES_FEW_NARROW 4  // the same for the 64-wide tiles
-#endif
-#ifndef MI355X_DMA_STAGES_MANY
-#define MI355X_DMA_STAGES_MANY 2  // ring depth otherwise (two workgroups per CU)
-#endif
+constexpr int kStagesFew = 4;   // ring depth when the tiles do not exceed the CUs
+constexpr int kStagesMany = 2;  // otherwise (two workgroups per CU)
 constexpr int kTileRows = 128;                          // activation rows per tile
 constexpr int kMaxBN = 160;                             // widest W tile (columns of the output tile)
 
@@ -56,7 +62,7 @@ constexpr int kMaxBN = 160;                             // widest W tile (column
 template <int BN, int J = 4>
 struct DmaGeo {
   static_assert(BN == 64 || BN == 128 || BN == 160, "tile width");
-  static_assert(J == 4 || J == 2, "tile rows");
+  static_assert(J == 4 || (J == 3 && BN != 160) || J == 2, "tile rows");
   static constexpr int kNI = BN / 32;                  // 16-column MFMA tiles per wave (2 x 2 waves)
   static constexpr int kRows = 32 * J;                 // activation rows of the tile
   static constexpr int kXOff = BN * 8;                 // uint4 offset of the activation tile
@@ -121,6 +127,7 @@ struct DmaSources {
   const float* as;    // activation scale of row m0, K group 0
   uint32_t woff[5];   // per-lane byte offsets from w of the W rows each DMA instruction fills
   uint32_t xoff[4];   // the same for the activation rows, from x (J of them)
+  uint32_t wback[5];  // KTAIL: how far the last K group's W reads step back into the row (chunks past K)
   uint32_t soff;      // per-lane byte offset from as of the scale this lane stages
   const float* ws_a;  // weight scales of the (at most two) 128-column blocks the wave's columns touch
   const float* ws_b;
@@ -135,21 +142,23 @@ __device__ __forceinline__ uint4* stage_ptr(uint4* ring) {
 }
 
 // DMA instruction d (0 .. kDmaPerStage-1) of a stage: W rows, then X rows, then scales.
-template <int BN, int S, int J = 4>
-__device__ __forceinline__ void issue_one(uint4* ring, const DmaSources& src, int64_t kb, int64_t as_sk, int wave,
-                                          int d) {
+template <int BN, int S, int J, bool KTAIL>
+__device__ __forceinline__ void issue_one(uint4* ring, const DmaSources& src, int64_t kb, int64_t KB, int64_t as_sk,
+                                          int wave, int d) {
   using G = DmaGeo<BN, J>;
   uint4* st = stage_ptr<BN, S, J>(ring);
   const int64_t koff = kb * kGroup;
-  if (d < G::kNI) dma16(src.w + koff, src.woff[d], st + (d * 4 + wave) * 64);
+  if (d < G::kNI)
+    dma16(src.w + koff, KTAIL && kb == KB - 1 ? src.woff[d] - src.wback[d] : src.woff[d], st + (d * 4 + wave) * 64);
   else if (d < G::kNI + J) dma16(src.x + koff, src.xoff[d - G::kNI], st + G::kXOff + ((d - G::kNI) * 4 + wave) * 64);
   else dma4(src.as + kb * as_sk, src.soff, reinterpret_cast<float*>(st + G::kScaleOff) + wave * 64);
 }
 
-template <int BN, int S, int J = 4>
-__device__ __forceinline__ void issue_stage(uint4* ring, const DmaSources& src, int64_t kb, int64_t as_sk, int wave) {
+template <int BN, int S, int J, bool KTAIL>
+__device__ __forceinline__ void issue_stage(uint4* ring, const DmaSources& src, int64_t kb, int64_t KB, int64_t as_sk,
+                                            int wave) {
 #pragma unroll
-  for (int d = 0; d < DmaGeo<BN, J>::kDmaPerStage; ++d) issue_one<BN, S, J>(ring, src, kb, as_sk, wave, d);
+  for (int d = 0; d < DmaGeo<BN, J>::kDmaPerStage; ++d) issue_one<BN, S, J, KTAIL>(ring, src, kb, KB, as_sk, wave, d);
 }
 
 // What the first MFMAs of a K step need, read from its stage one step early: the four
@@ -212,7 +221,7 @@ __device__ __forceinline__ void fold_tile(v4f (&acc)[BN / 32][J], const v4f (&p)
 //   is refilled with K group kb+STAGES, and the last weight fragments are multiplied.
 // The LDS reads of each part so run behind MFMAs that do not depend on them.  Every
 // output element is still folded once per K group, in K order.
-template <int BN, int STAGES, int CUR, int J = 4>
+template <int BN, int STAGES, int CUR, int J, bool KTAIL>
 __device__ __forceinline__ void k_step(uint4* ring, v4f (&acc)[BN / 32][J], StepHead<BN, J>& h, const DmaSources& src,
                                        int64_t kb, int64_t KB, int64_t as_sk, int64_t ws_sk, int wave, int wm,
                                        int wn, int r, int g) {
@@ -267,7 +276,7 @@ __device__ __forceinline__ void k_step(uint4* ring, v4f (&acc)[BN / 32][J], Step
     const int i = NA + t / J, j = t % J;
     p[i][j] = mfma_16x16x128_e4m3(a[i], h.b[j]);
 #pragma unroll
-    for (int d = t * ND / NM; d < (t + 1) * ND / NM; ++d) issue_one<BN, CUR, J>(ring, src, ahead, as_sk, wave, d);
+    for (int d = t * ND / NM; d < (t + 1) * ND / NM; ++d) issue_one<BN, CUR, J, KTAIL>(ring, src, ahead, KB, as_sk, wave, d);
     if (j == J - 1 && i > 0) fold_tile<BN, J>(acc, p[i - 1], sa, sb, src.use_b, i - 1);
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -276,12 +285,94 @@ __device__ __forceinline__ void k_step(uint4* ring, v4f (&acc)[BN / 32][J], Step
   h = nh;
 }
 
-template <int STAGES, int BN, typename OutT, int J = 4>
+// The fragments of one K group in registers: what all of its MFMAs need.
+template <int BN, int J>
+struct StepRegs {
+  v8i a[BN / 32], b[J];
+  float as_v[J];
+  float wa, wb;
+};
+
+// Reads fragment f of stage S's K group: the J activation fragments, then the BN / 32 weight
+// fragments.
+template <int BN, int S, int J>
+__device__ __forceinline__ void read_frag(const uint4* ring, StepRegs<BN, J>& h, int f, int wm, int wn, int r, int g) {
+  using G = DmaGeo<BN, J>;
+  const uint4* st = ring + S * G::kStageU4;
+  if (f < J) {
+    const int row = wm * 16 * J + 16 * f + r;
+    h.b[f] = pack_v8i(st[G::kXOff + row * 8 + (g ^ (row & 7))], st[G::kXOff + row * 8 + ((g + 4) ^ (row & 7))]);
+  } else {
+    h.a[f - J] = read_a<BN, S, J>(ring, f - J, wn, r, g);
+  }
+}
+template <int BN, int S, int J>
+__device__ __forceinline__ void read_scales(const uint4* ring, StepRegs<BN, J>& h, const DmaSources& src, int64_t kb,
+                                            int64_t ws_sk, int wm, int r) {
+  const float* sc_lds = reinterpret_cast<const float*>(ring + S * DmaGeo<BN, J>::kStageU4 + DmaGeo<BN, J>::kScaleOff);
+#pragma unroll
+  for (int j = 0; j < J; ++j) h.as_v[j] = sc_lds[wm * 16 * J + 16 * j + r];
+  h.wa = src.ws_a[kb * ws_sk];
+  h.wb = src.ws_b[kb * ws_sk];
+}
+
+// One K group kb whose fragments f were read during the previous step (the form with one
+// workgroup per CU, where a wave has 512 registers).  While its MFMAs run, the next group's
+// fragments are read from stage CUR + 1 into nf, and stage CUR, which every wave had read
+// before the last barrier, is refilled with K group kb + STAGES.  Both go out between the
+// MFMAs, and the fold of a 16x16 tile two MFMAs after its own, so neither the LDS reads nor
+// the MFMA latency stand in the chain.
+template <int BN, int STAGES, int CUR, int J, bool KTAIL>
+__device__ __forceinline__ void reg_step(uint4* ring, v4f (&acc)[BN / 32][J], const StepRegs<BN, J>& f,
+                                         StepRegs<BN, J>& nf, const DmaSources& src, int64_t kb, int64_t KB,
+                                         int64_t as_sk, int64_t ws_sk, int wave, int wm, int wn, int r, int g) {
+  using G = DmaGeo<BN, J>;
+  constexpr int NI = G::kNI, NM = NI * J, NF = NI + J, ND = G::kDmaPerStage;
+  constexpr int NXT = (CUR + 1) % STAGES;
+  const int64_t nkb = kb + 1 < KB ? kb + 1 : KB - 1;
+  const int64_t ahead = kb + STAGES < KB ? kb + STAGES : KB - 1;
+  float sa[J], sb[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    sa[j] = f.as_v[j] * f.wa;
+    sb[j] = BN == 160 ? f.as_v[j] * f.wb : sa[j];
+  }
+  read_scales<BN, NXT, J>(ring, nf, src, nkb, ws_sk, wm, r);
+  constexpr int kLag = 2;
+  v4f p[kLag + 1];
+  auto fold = [&](int t) {
+    const int i = t / J, j = t % J;
+    const float sc = (BN == 160 && ((src.use_b >> i) & 1)) ? sb[j] : sa[j];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[i][j][v] = __builtin_fmaf(p[t % (kLag + 1)][v], sc, acc[i][j][v]);
+  };
+#pragma unroll
+  for (int t = 0; t < NM; ++t) {
+    p[t % (kLag + 1)] = mfma_16x16x128_e4m3(f.a[t / J], f.b[t % J]);
+#pragma unroll
+    for (int d = t * ND / NM; d < (t + 1) * ND / NM; ++d) issue_one<BN, CUR, J, KTAIL>(ring, src, ahead, KB, as_sk, wave, d);
+    // The fragments of the next group over the first three quarters of the MFMAs.
+    constexpr int NR = NM * 3 / 4 > 0 ? NM * 3 / 4 : 1;
+    if (t < NR) {
+#pragma unroll
+      for (int x = t * NF / NR; x < (t + 1) * NF / NR; ++x) read_frag<BN, NXT, J>(ring, nf, x, wm, wn, r, g);
+    }
+    if (t >= kLag) fold(t - kLag);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int t = NM - kLag; t < NM; ++t) fold(t);
+  wait_vm_lgkm0<ND * (STAGES - 2)>();
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <int STAGES, int BN, typename OutT, int J, bool KTAIL>
 __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dma_kernel(
     const uint8_t* __restrict__ q, int64_t ldq, const float* __restrict__ as, int64_t as_sk,
     const uint8_t* __restrict__ w, int64_t ldw, const float* __restrict__ ws, int64_t ws_sn,
     int64_t ws_sk, uint16_t* __restrict__ out, int64_t ldo, int64_t M, int64_t N, int64_t KB,
-    int64_t tiles_m, int64_t tiles_n, int vec_out) {
+    int64_t tiles_m, int64_t tiles_n, int vec_out, int tail) {
   __shared__ uint4 ring[STAGES * DmaGeo<BN, J>::kStageU4];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -307,6 +398,9 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
     const int c = (lane & 7) ^ (rr & 7);
     const int64_t wrow = (n0 + rr) < N ? rr : (N - 1 - n0);
     src.woff[i] = static_cast<uint32_t>(wrow * ldw + 16 * c);
+    // Chunks of the last group past K read the group's first chunk of the same row: the
+    // activation codes there are zero, and a NaN code can only come from the row itself.
+    if (KTAIL) src.wback[i] = 16 * c >= tail ? 16 * c : 0;
     if (i < J) {
       const int64_t xrow = (m0 + rr) < M ? rr : (M - 1 - m0);
       src.xoff[i] = static_cast<uint32_t>(xrow * ldq + 16 * c);
@@ -315,7 +409,7 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
   {
     // Wave w stages the scales of tile rows 64 (w & 1) .. +63 (waves 2, 3 duplicate 0, 1); a
     // 64-row tile's are staged by every wave alike.
-    const int64_t srow = (J == 4 ? (wave & 1) * 64 : 0) + lane;
+    const int64_t srow = (J >= 3 ? (wave & 1) * 64 : 0) + lane;
     src.soff = static_cast<uint32_t>(4 * (m0 + srow < M ? srow : M - 1 - m0));
   }
   {
@@ -339,39 +433,49 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
 #pragma unroll
     for (int j = 0; j < J; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
-  static_assert(STAGES >= 2 && STAGES <= 6, "stages");
-  issue_stage<BN, 0, J>(ring, src, 0, as_sk, wave);
-  issue_stage<BN, 1, J>(ring, src, KB > 1 ? 1 : KB - 1, as_sk, wave);
-  if constexpr (STAGES >= 3) issue_stage<BN, 2, J>(ring, src, KB > 2 ? 2 : KB - 1, as_sk, wave);
-  if constexpr (STAGES >= 4) issue_stage<BN, 3, J>(ring, src, KB > 3 ? 3 : KB - 1, as_sk, wave);
-  if constexpr (STAGES >= 5) issue_stage<BN, 4, J>(ring, src, KB > 4 ? 4 : KB - 1, as_sk, wave);
-  if constexpr (STAGES >= 6) issue_stage<BN, 5, J>(ring, src, KB > 5 ? 5 : KB - 1, as_sk, wave);
+  static_assert(STAGES == 2 || STAGES == 4, "stages");
+  issue_stage<BN, 0, J, KTAIL>(ring, src, 0, KB, as_sk, wave);
+  issue_stage<BN, 1, J, KTAIL>(ring, src, KB > 1 ? 1 : KB - 1, KB, as_sk, wave);
+  if constexpr (STAGES == 4) {
+    issue_stage<BN, 2, J, KTAIL>(ring, src, KB > 2 ? 2 : KB - 1, KB, as_sk, wave);
+    issue_stage<BN, 3, J, KTAIL>(ring, src, KB > 3 ? 3 : KB - 1, KB, as_sk, wave);
+  }
   wait_vm_lgkm0<G::kDmaPerStage * (STAGES - 1)>();
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  StepHead<BN, J> h;
-  read_head<BN, 0, J>(ring, h, src, 0, ws_sk, wm, wn, r, g);
   int64_t kb = 0;
-#define MI355X_KSTEP(S, KBV) k_step<BN, STAGES, S, J>(ring, acc, h, src, KBV, KB, as_sk, ws_sk, wave, wm, wn, r, g)
-  for (; kb + STAGES <= KB; kb += STAGES) {
-    MI355X_KSTEP(0, kb);
-    MI355X_KSTEP(1, kb + 1);
-    if constexpr (STAGES >= 3) MI355X_KSTEP(2, kb + 2);
-    if constexpr (STAGES >= 4) MI355X_KSTEP(3, kb + 3);
-    if constexpr (STAGES >= 5) MI355X_KSTEP(4, kb + 4);
-    if constexpr (STAGES >= 6) MI355X_KSTEP(5, kb + 5);
-  }
-  // The last KB % STAGES groups.
-  if (kb < KB) MI355X_KSTEP(0, kb);
-  if constexpr (STAGES >= 3)
-    if (kb + 1 < KB) MI355X_KSTEP(1, kb + 1);
-  if constexpr (STAGES >= 4)
-    if (kb + 2 < KB) MI355X_KSTEP(2, kb + 2);
-  if constexpr (STAGES >= 5)
-    if (kb + 3 < KB) MI355X_KSTEP(3, kb + 3);
-  if constexpr (STAGES >= 6)
-    if (kb + 4 < KB) MI355X_KSTEP(4, kb + 4);
+  if constexpr (STAGES == 2) {
+    StepHead<BN, J> h;
+    read_head<BN, 0, J>(ring, h, src, 0, ws_sk, wm, wn, r, g);
+#define MI355X_KSTEP(S, KBV) k_step<BN, STAGES, S, J, KTAIL>(ring, acc, h, src, KBV, KB, as_sk, ws_sk, wave, wm, wn, r, g)
+    for (; kb + 2 <= KB; kb += 2) {
+      MI355X_KSTEP(0, kb);
+      MI355X_KSTEP(1, kb + 1);
+    }
+    if (kb < KB) MI355X_KSTEP(0, kb);
 #undef MI355X_KSTEP
+  } else {
+    StepRegs<BN, J> f0, f1;
+    read_scales<BN, 0, J>(ring, f0, src, 0, ws_sk, wm, r);
+#pragma unroll
+    for (int x = 0; x < NI + J; ++x) read_frag<BN, 0, J>(ring, f0, x, wm, wn, r, g);
+    wait_vm_lgkm0<G::kDmaPerStage * (STAGES - 2)>();  // stage 1 landed, stage 0 read by this wave
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#define MI355X_KSTEP(S, F, NF, KBV) \
+  reg_step<BN, STAGES, S, J, KTAIL>(ring, acc, F, NF, src, KBV, KB, as_sk, ws_sk, wave, wm, wn, r, g)
+    for (; kb + STAGES <= KB; kb += STAGES) {
+      MI355X_KSTEP(0, f0, f1, kb);
+      MI355X_KSTEP(1, f1, f0, kb + 1);
+      MI355X_KSTEP(2, f0, f1, kb + 2);
+      MI355X_KSTEP(3, f1, f0, kb + 3);
+    }
+    // The last KB % STAGES groups.
+    if (kb < KB) MI355X_KSTEP(0, f0, f1, kb);
+    if (kb + 1 < KB) MI355X_KSTEP(1, f1, f0, kb + 1);
+    if (kb + 2 < KB) MI355X_KSTEP(2, f0, f1, kb + 2);
+#undef MI355X_KSTEP
+  }
   wait_vm_lgkm0<0>();  // no DMA may still target LDS when the workgroup ends
 
   if (vec_out == 2) {
@@ -444,11 +548,12 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
 }  // namespace
 
 bool tile_dma_supported(const uint8_t* q, int64_t ldq, int64_t as_sm, int64_t as_sk, const uint8_t* w,
-                        int64_t ldw, int64_t M, int64_t K) {
+                        int64_t ldw, int64_t M, int64_t K, bool q_padded) {
   // The per-lane DMA offsets within a tile are 32-bit (the row bases are 64-bit).
   constexpr int64_t kMaxOff = 0xffffffffLL - kGroup;
   if (ldq > kMaxOff / (kTileRows - 1) || ldw > kMaxOff / (kMaxBN - 1)) return false;
-  return K % kGroup == 0 && ldq % 16 == 0 && ldw % 16 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0 &&
+  const bool k_ok = K % kGroup == 0 || (q_padded && K % 16 == 0);
+  return k_ok && ldq % 16 == 0 && ldw % 16 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0 &&
          reinterpret_cast<uintptr_t>(w) % 16 == 0 && as_sm == 1 && as_sk >= M;
 }
 
@@ -456,48 +561,45 @@ int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_s
                     int64_t ldw, const float* ws, int64_t ws_sn, int64_t ws_sk, void* out, int out_dtype,
                     int64_t ldo, int64_t M, int64_t N, int64_t K, int bn, int rows, hipStream_t stream) {
   if (bn != 64 && bn != 128 && bn != 160) return MI355X_FP8_ERR_INVALID;
-  if (rows != 128 && (rows != 64 || bn == 160)) return MI355X_FP8_ERR_INVALID;
+  if (rows != 128 && ((rows != 64 && rows != 96) || bn == 160)) return MI355X_FP8_ERR_INVALID;
   const int64_t tiles_m = (M + rows - 1) / rows;
   const int64_t tiles_n = (N + bn - 1) / bn;
   if (tiles_m * tiles_n > 0x7fffffffLL) return MI355X_FP8_ERR_UNSUPPORTED;
   const int vec_out = out_vec_mode(out, ldo);
   dim3 grid(static_cast<unsigned>(tiles_m * tiles_n));
+  const int tail = static_cast<int>(K % kGroup);
   uint16_t* o = static_cast<uint16_t*>(out);
-  // Two stages (76 KiB, room for the 160-wide W tile) let two workgroups share a CU.
-  // When the tiles do not fill the CUs anyway, each K step waits on its DMA round trip,
-  // so a deeper ring (one workgroup per CU) keeps more K groups in flight: three stages,
-  // four for the 64-wide tiles, whose short steps wait longest (measured on o_proj and down
-  // at 256 and 536 rows; four stages for the wider tiles measured slower).
+  // Two stages (76 KiB, room for the 160-wide W tile) let two workgroups share a CU.  When the
+  // tiles do not fill the CUs anyway, four stages (one workgroup per CU) keep more K groups in
+  // flight; six, where they fit, measured the same (28.0 and 28.3 us for N = 2560, K = 9728 at
+  // 536 rows).  64x64 tiles have room for two workgroups of four stages.
   const bool few = tiles_m * tiles_n <= device_cus();
-#define MI355X_DMA_ARGS q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, o, ldo, M, N, K / kGroup, tiles_m, tiles_n, vec_out
-#define MI355X_DMA_LAUNCH(ST, BN)                                                                                  \
-  (out_dtype == kBF16 ? tile_gemm_dma_kernel<ST, BN, bf16_t><<<grid, kDmaThreads, 0, stream>>>(MI355X_DMA_ARGS) \
-                      : tile_gemm_dma_kernel<ST, BN, f16_t><<<grid, kDmaThreads, 0, stream>>>(MI355X_DMA_ARGS))
-#define MI355X_DMA_LAUNCH64(ST, BN)                                                                                   \
-  (out_dtype == kBF16 ? tile_gemm_dma_kernel<ST, BN, bf16_t, 2><<<grid, kDmaThreads, 0, stream>>>(MI355X_DMA_ARGS) \
-                      : tile_gemm_dma_kernel<ST, BN, f16_t, 2><<<grid, kDmaThreads, 0, stream>>>(MI355X_DMA_ARGS))
+#define MI355X_DMA_ARGS q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, o, ldo, M, N, (K + kGroup - 1) / kGroup, tiles_m, tiles_n, vec_out, tail
+#define MI355X_DMA_LAUNCH_K(ST, BN, J, KT)                                                                            \
+  (out_dtype == kBF16 ? tile_gemm_dma_kernel<ST, BN, bf16_t, J, KT><<<grid, kDmaThreads, 0, stream>>>(MI355X_DMA_ARGS) \
+                      : tile_gemm_dma_kernel<ST, BN, f16_t, J, KT><<<grid, kDmaThreads, 0, stream>>>(MI355X_DMA_ARGS))
+#define MI355X_DMA_LAUNCH(ST, BN, J) \
+  (tail == 0 ? MI355X_DMA_LAUNCH_K(ST, BN, J, false) : MI355X_DMA_LAUNCH_K(ST, BN, J, true))
+#define MI355X_DMA_ROWS(BN, J)                              \
+  do {                                                      \
+    if (few) MI355X_DMA_LAUNCH(kStagesFew, BN, J);          \
+    else MI355X_DMA_LAUNCH(kStagesMany, BN, J);             \
+  } while (0)
   if (rows == 64) {
-    // 64-row tiles (half the activation rows of a tile, J = 2): for row counts just past a
-    // multiple of 64 whose 128-row tiles leave CUs idle.  Two workgroups per CU share it when
-    // the tiles outnumber the CUs.
-    if (!few) {
-      if (bn == 64) MI355X_DMA_LAUNCH64(MI355X_DMA_STAGES_MANY, 64);
-      else MI355X_DMA_LAUNCH64(MI355X_DMA_STAGES_MANY, 128);
-    } else {
-      if (bn == 64) MI355X_DMA_LAUNCH64(MI355X_DMA_STAGES_FEW_NARROW, 64);
-      else MI355X_DMA_LAUNCH64(MI355X_DMA_STAGES_FEW, 128);
-    }
-  } else if (!few) {
-    if (bn == 160) MI355X_DMA_LAUNCH(MI355X_DMA_STAGES_MANY, 160);
-    else if (bn == 64) MI355X_DMA_LAUNCH(MI355X_DMA_STAGES_MANY, 64);
-    else MI355X_DMA_LAUNCH(MI355X_DMA_STAGES_MANY, 128);
+    if (bn == 64) MI355X_DMA_LAUNCH(kStagesFew, 64, 2);
+    else MI355X_DMA_ROWS(128, 2);
+  } else if (rows == 96) {
+    if (!few) return MI355X_FP8_ERR_INVALID;
+    if (bn == 64) MI355X_DMA_LAUNCH(kStagesFew, 64, 3);
+    else MI355X_DMA_LAUNCH(kStagesFew, 128, 3);
   } else {
-    if (bn == 160) MI355X_DMA_LAUNCH(MI355X_DMA_STAGES_FEW, 160);
-    else if (bn == 64) MI355X_DMA_LAUNCH(MI355X_DMA_STAGES_FEW_NARROW, 64);
-    else MI355X_DMA_LAUNCH(MI355X_DMA_STAGES_FEW, 128);
+    if (bn == 160) MI355X_DMA_ROWS(160, 4);
+    else if (bn == 64) MI355X_DMA_ROWS(64, 4);
+    else MI355X_DMA_ROWS(128, 4);
   }
-#undef MI355X_DMA_LAUNCH64
+#undef MI355X_DMA_ROWS
 #undef MI355X_DMA_LAUNCH
+#undef MI355X_DMA_LAUNCH_K
 #undef MI355X_DMA_ARGS
   return hipGetLastError() == hipSuccess ? MI355X_FP8_OK : MI355X_FP8_ERR_LAUNCH;
 }
