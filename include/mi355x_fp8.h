@@ -109,6 +109,20 @@ int mi355x_fp8_block_gemm(const uint8_t* q, int64_t ldq, const float* as, int64_
                           int64_t M, int64_t N, int64_t K, void* workspace,
                           size_t workspace_bytes, int config, void* stream);
 
+/*
+ * Block GEMM on a merged gate/up weight (N = 2 I rows, gate rows first) with SiLU(gate) * up in
+ * its epilogue, at prefill sizes: h[M, I] bf16 = bf16(bf16(silu(g)) * u) on the bf16 gate and up
+ * outputs g, u that mi355x_fp8_block_gemm would write (same bits).  Replaces the merged gate_up
+ * projection's GEMM and silu_mul (engine/kernels/fused.py:127-137, 217-232).  Operands as in
+ * mi355x_fp8_block_gemm; returns MI355X_FP8_ERR_UNSUPPORTED, having launched nothing, when the
+ * call does not fit the prefill kernels (decode sizes, K not a multiple of 128, N not a multiple
+ * of 32, activation scales not K-group-major, unaligned operands or h rows), and the caller then
+ * runs the two steps.
+ */
+int mi355x_fp8_block_gemm_silu(const uint8_t* q, int64_t ldq, const float* as, int64_t as_sm, int64_t as_sk,
+                               const uint8_t* w, int64_t ldw, const float* ws, int64_t ws_sn, int64_t ws_sk, void* h,
+                               int64_t ldh, int64_t M, int64_t N, int64_t K, void* stream);
+
 /* Workspace bytes that mi355x_fp8_linear needs: the quantized activations, their scales
  * and the GEMM's workspace.  Same rules as the GEMM workspace. */
 size_t mi355x_fp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int config);

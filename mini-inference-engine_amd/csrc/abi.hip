@@ -193,6 +193,16 @@ int mi355x_fp8_block_gemm(const uint8_t* q, int64_t ldq, const float* as, int64_
                            ldo, M, N, K, workspace, static_cast<hipStream_t>(stream));
 }
 
+int mi355x_fp8_block_gemm_silu(const uint8_t* q, int64_t ldq, const float* as, int64_t as_sm, int64_t as_sk,
+                               const uint8_t* w, int64_t ldw, const float* ws, int64_t ws_sn, int64_t ws_sk, void* h,
+                               int64_t ldh, int64_t M, int64_t N, int64_t K, void* stream) {
+  if (M < 0 || N < 0 || N % 2 != 0 || K <= 0 || ldq < K || ldw < K || ldh < N / 2) return MI355X_FP8_ERR_INVALID;
+  if (M == 0 || N == 0) return MI355X_FP8_OK;
+  if (!q || !as || !w || !ws || !h) return MI355X_FP8_ERR_INVALID;
+  return launch_gate_up_silu(q, ldq, as, as_sm, as_sk, w, ldw, ws, ws_sn, ws_sk, static_cast<uint16_t*>(h), ldh, M, N,
+                             K, static_cast<hipStream_t>(stream));
+}
+
 size_t mi355x_fp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int config) {
   LinearLayout L;
   if (M < 0 || N < 0 || K <= 0 || linear_layout(M, N, K, config, &L) != MI355X_FP8_OK) return 0;

@@ -603,8 +603,7 @@ __global__ __launch_bounds__(kStreamWaves * 64) void stream_gemm_kernel(
       const float* sfu = scl + (2 + ((n_rows + n0 + nl) / kGroup != nbu0 ? 1 : 0)) * kTokS + tok;
       const float g = bf16_bits_val(OutCvt<bf16_t>::cvt(fold(pf, sf)));
       const float u = bf16_bits_val(OutCvt<bf16_t>::cvt(fold(pf + 16 * kHalfT, sfu)));
-      const float silu = round_bf16(g / (1.0f + expf(-g)));
-      out[(m_base + tok) * ldo + n0 + nl] = f32_to_bf16_bits(silu * u);
+      out[(m_base + tok) * ldo + n0 + nl] = silu_mul_bf16(g, u);
     } else {
       const float acc = fold(pf, sf);
       if (RAGGED || n0 + nl < N) out[(m_base + tok) * ldo + n0 + nl] = OutCvt<OutT>::cvt(acc);
@@ -851,7 +850,7 @@ int64_t device_cus() {
 // A last, partly filled wave costs 0.7 + 0.3 x its fill of a full one (a half-filled wave
 // measured 0.75-0.98).  Every kernel gives the same bits, so the choice may follow M.
 // (The figures rank the tiles; the 128-row kernel's single waves have since become 10-20 % faster
-// in the same order, and launch_block_gemm shortens its tiles to 96 rows where those fit.)
+// in the same order, and prefill_tile shortens its tiles to 96 rows where those fit.)
 namespace {
 struct TileVariant {
   int rows, bn;
@@ -895,6 +894,19 @@ PrefillChoice choose_prefill(int64_t M, int64_t N, int64_t cus, bool rows256_ok)
     }
   }
   return best;
+}
+
+// The tile that is launched: the model's choice, 128-row tiles in 96 rows where those still fit
+// one per CU: more CUs share the rows, and a tile's serial K loop has a quarter less to multiply
+// and a sixth less to load per step.
+// Measured 128 against 96 rows (us, weights from HBM, N = 2560): 64 wide, K = 9728 at 512
+// rows 34.1 / 26.9, at 536 27.9 / 27.6, K = 4096 at 536 12.6 / 12.2; 128 wide, K = 4096 at
+// 1024 rows 21.3 / 18.4, K = 9728 48.3 / 41.1.
+PrefillChoice prefill_tile(int64_t M, int64_t N, bool rows256_ok) {
+  const int64_t cus = device_cus();
+  PrefillChoice c = choose_prefill(M, N, cus, rows256_ok);
+  if (c.rows == 128 && c.bn <= 128 && cdiv(M, 96) * cdiv(N, c.bn) <= cus) c.rows = 96;
+  return c;
 }
 }  // namespace
 
@@ -999,6 +1011,24 @@ static int launch_typed(const GemmPlan& plan, const uint8_t* q, int64_t ldq, con
   return hipGetLastError() == hipSuccess ? MI355X_FP8_OK : MI355X_FP8_ERR_LAUNCH;
 }
 
+// The prefill kernels on a merged gate/up weight with SiLU(gate) * up applied in the epilogue.
+int launch_gate_up_silu(const uint8_t* q, int64_t ldq, const float* as, int64_t as_sm, int64_t as_sk,
+                        const uint8_t* w, int64_t ldw, const float* ws, int64_t ws_sn, int64_t ws_sk, uint16_t* h,
+                        int64_t ldh, int64_t M, int64_t N, int64_t K, hipStream_t stream) {
+  GemmPlan plan;
+  const int st = plan_gemm(M, N, K, MI355X_FP8_CONFIG_AUTO, &plan);
+  if (st != MI355X_FP8_OK) return st;
+  // The prefill tiles only (the stream kernel has no paired form), h rows of 16-byte pieces, and
+  // halves that start on a 16-column MFMA tile.
+  if (plan.kernel != MI355X_FP8_CONFIG_TILE128 || N % 32 != 0 || K % kGroup != 0 || out_vec_mode(h, ldh) != 2 ||
+      !tile_dma_supported(q, ldq, as_sm, as_sk, w, ldw, M, K, false) || (N / 2 + 256) * ldw > 0xffffffffLL)
+    return MI355X_FP8_ERR_UNSUPPORTED;
+  const PrefillChoice c = prefill_tile(M, N, tile256_offsets_ok(ldq, ldw, M, N, K));
+  if (c.rows > 128)
+    return launch_tile256(q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, h, kBF16, ldh, M, N, K, c.bn, c.rows, stream, true);
+  return launch_tile_dma(q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, h, kBF16, ldh, M, N, K, c.bn, c.rows, stream, true);
+}
+
 int launch_block_gemm(const GemmPlan& plan, const uint8_t* q, int64_t ldq, const float* as,
                       int64_t as_sm, int64_t as_sk, const uint8_t* w, int64_t ldw, const float* ws,
                       int64_t ws_sn, int64_t ws_sk, void* out, int out_dtype, int64_t ldo,
@@ -1027,14 +1057,7 @@ int launch_block_gemm(const GemmPlan& plan, const uint8_t* q, int64_t ldq, const
                           tile256_width(M, N, device_cus()), 256, stream);
   }
   if (plan.kernel == MI355X_FP8_CONFIG_TILE128 && dma_ok) {
-    const int64_t cus = device_cus();
-    PrefillChoice c = choose_prefill(M, N, cus, whole && tile256_offsets_ok(ldq, ldw, M, N, K));
-    // 128-row tiles in 96 rows where those still fit one per CU: more CUs share the rows, and a
-    // tile's serial K loop has a quarter less to multiply and a sixth less to load per step.
-    // Measured 128 against 96 rows (us, weights from HBM, N = 2560): 64 wide, K = 9728 at 512
-    // rows 34.1 / 26.9, at 536 27.9 / 27.6, K = 4096 at 536 12.6 / 12.2; 128 wide, K = 4096 at
-    // 1024 rows 21.3 / 18.4, K = 9728 48.3 / 41.1.
-    if (c.rows == 128 && c.bn <= 128 && cdiv(M, 96) * cdiv(N, c.bn) <= cus) c.rows = 96;
+    const PrefillChoice c = prefill_tile(M, N, whole && tile256_offsets_ok(ldq, ldw, M, N, K));
     if (c.rows > 128)
       return launch_tile256(q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, out, out_dtype, ldo, M, N, K, c.bn, c.rows,
                             stream);

@@ -45,6 +45,12 @@ int launch_block_gemm(const GemmPlan& plan, const uint8_t* q, int64_t ldq, const
                       int64_t ws_sn, int64_t ws_sk, void* out, int out_dtype, int64_t ldo,
                       int64_t M, int64_t N, int64_t K, void* workspace, hipStream_t stream);
 
+// Block GEMM on a merged gate/up weight with SiLU(gate) * up in the prefill kernels' epilogue:
+// h[M, N / 2] bf16; MI355X_FP8_ERR_UNSUPPORTED (nothing launched) when the call does not fit.
+int launch_gate_up_silu(const uint8_t* q, int64_t ldq, const float* as, int64_t as_sm, int64_t as_sk,
+                        const uint8_t* w, int64_t ldw, const float* ws, int64_t ws_sn, int64_t ws_sk, uint16_t* h,
+                        int64_t ldh, int64_t M, int64_t N, int64_t K, hipStream_t stream);
+
 // The whole linear in one stream-kernel launch (quantization inside), for plans of the stream
 // kernel with one token tile; MI355X_FP8_ERR_UNSUPPORTED (nothing launched) when the call
 // does not fit that form.
@@ -74,7 +80,12 @@ bool tile_dma_supported(const uint8_t* q, int64_t ldq, int64_t as_sm, int64_t as
 // bn: tile width, 64, 128 or 160; rows: tile rows, 128, or 96 or 64 (widths 64 and 128).
 int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_sk, const uint8_t* w,
                     int64_t ldw, const float* ws, int64_t ws_sn, int64_t ws_sk, void* out, int out_dtype,
-                    int64_t ldo, int64_t M, int64_t N, int64_t K, int bn, int rows, hipStream_t stream);
+                    int64_t ldo, int64_t M, int64_t N, int64_t K, int bn, int rows, hipStream_t stream,
+                    bool silu = false);
+
+// silu (both prefill kernels): w is a merged gate/up weight (N / 2 gate rows, then as many up
+// rows), a tile owns BN / 2 gate columns and the matching up columns, and out receives
+// silu_mul(gate, up) [M, N / 2] (bf16, out_vec_mode 2, N % 32 == 0, (N / 2 + 256) ldw < 2^32).
 
 // 256-row-tile prefill kernel (tile_gemm_256.hip), or its 192-row form (rows = 192); same
 // preconditions as the DMA kernel.  bn: tile width, 256, 224 or 192 (two-stage LDS ring) or
@@ -82,7 +93,8 @@ int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_s
 // measured cost on `cus` CUs.
 int launch_tile256(const uint8_t* q, int64_t ldq, const float* as, int64_t as_sk, const uint8_t* w,
                    int64_t ldw, const float* ws, int64_t ws_sn, int64_t ws_sk, void* out, int out_dtype,
-                   int64_t ldo, int64_t M, int64_t N, int64_t K, int bn, int rows, hipStream_t stream);
+                   int64_t ldo, int64_t M, int64_t N, int64_t K, int bn, int rows, hipStream_t stream,
+                    bool silu = false);
 int tile256_width(int64_t M, int64_t N, int64_t cus);
 // The prefill kernel the automatic dispatch picks for an M x N output on `cus` CUs (when the
 // LDS-DMA preconditions hold and the offsets fit): tile rows (64, 128, 192 or 256) and width.

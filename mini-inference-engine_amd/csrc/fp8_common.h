@@ -79,6 +79,32 @@ __device__ __forceinline__ float round_bf16(float f) {
   return __uint_as_float(static_cast<uint32_t>(f32_to_bf16_bits(f)) << 16);
 }
 
+// The reference's silu_mul on bf16 gate and up values (engine/kernels/fused.py:127-137):
+// silu = bf16(g / (1 + exp(-g))), then the bf16 product's bits.
+__device__ __forceinline__ uint16_t silu_mul_bf16(float g, float u) {
+  return f32_to_bf16_bits(round_bf16(g / (1.0f + expf(-g))) * u);
+}
+// Eight of them: two 16-byte pieces of gate and up columns in, one of h out.
+__device__ __forceinline__ uint4 silu_mul8(uint4 gate, uint4 up) {
+  const uint32_t gw[4] = {gate.x, gate.y, gate.z, gate.w}, uw[4] = {up.x, up.y, up.z, up.w};
+  uint32_t h[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    h[i] = silu_mul_bf16(__uint_as_float(gw[i] << 16), __uint_as_float(uw[i] << 16)) |
+           (static_cast<uint32_t>(silu_mul_bf16(__uint_as_float(gw[i] & 0xffff0000u), __uint_as_float(uw[i] & 0xffff0000u))) << 16);
+  return make_uint4(h[0], h[1], h[2], h[3]);
+}
+// Stores 8 consecutive 16-bit values at dst, columns [n, n + 8) of end.
+__device__ __forceinline__ void store8_cols(uint16_t* dst, uint4 v, int64_t n, int64_t end) {
+  if (n + 8 <= end) {
+    store16_nt(dst, v);
+  } else {
+    const uint16_t* hv = reinterpret_cast<const uint16_t*>(&v);
+    for (int i = 0; i < 8; ++i)
+      if (n + i < end) dst[i] = hv[i];
+  }
+}
+
 // Two fp32 -> two OCP e4m3fn codes (round-to-nearest-even), packed into the low 16 bits.
 __device__ __forceinline__ uint32_t cvt_pk_e4m3(float a, float b) {
   return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false)) & 0xffffu;

@@ -58,8 +58,7 @@ __global__ __launch_bounds__(kSmqThreads) void silu_mul_quant_kernel(
   uint16_t hb[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const float silu = round_bf16(gv[i] / (1.0f + expf(-gv[i])));
-    hb[i] = f32_to_bf16_bits(silu * uv[i]);
+    hb[i] = silu_mul_bf16(gv[i], uv[i]);
     t[i] = __uint_as_float(static_cast<uint32_t>(hb[i]) << 16);
   }
   uint32_t packed[2];

@@ -40,6 +40,9 @@
 // The output tile leaves through LDS as full-row 16-byte non-temporal stores when the output
 // rows are 16-byte aligned (staged_index, fp8_common.h), else straight from the registers.
 //
+// SILU: as in the 256-row kernel, a tile owns BN / 2 gate and the matching up columns of a merged
+// weight and writes silu(gate) * up (two decode layers at 32 rows 155 -> 146 us).
+//
 // Preconditions (checked by the launcher): K % 128 == 0 (% 16 with padded codes), W/q base pointers and leading
 // dimensions 16-byte aligned, activation scales K-group-major (as_sm == 1) with row
 // length as_sk >= M, row strides below 2^32 / 159 bytes (W) and 2^32 / 127 bytes (q), so that
@@ -198,13 +201,13 @@ __device__ __forceinline__ void read_head(const uint4* ring, StepHead<BN, J>& h,
 }
 
 // Folds column tile i's partials into the accumulator: acc = fma(p, as * ws, acc), ws being
-// the scale of the 128-column weight block the tile lies in.  Only BN = 160 lets a wave's
-// tiles straddle two blocks; the step forms both blocks' four products once (sa, sb), and each
+// the scale of the 128-column weight block the tile lies in.  TWO: the wave's
+// tiles may straddle two blocks; the step forms both blocks' four products once (sa, sb), and each
 // tile picks its block's set on the scalar unit.
-template <int BN, int J = 4>
+template <int BN, int J, bool TWO>
 __device__ __forceinline__ void fold_tile(v4f (&acc)[BN / 32][J], const v4f (&p)[J], const float (&sa)[J],
                                           const float (&sb)[J], uint32_t use_b, int i) {
-  const bool ub = BN == 160 && ((use_b >> i) & 1);
+  const bool ub = TWO && ((use_b >> i) & 1);
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     const float sc = ub ? sb[j] : sa[j];
@@ -221,7 +224,7 @@ __device__ __forceinline__ void fold_tile(v4f (&acc)[BN / 32][J], const v4f (&p)
 //   is refilled with K group kb+STAGES, and the last weight fragments are multiplied.
 // The LDS reads of each part so run behind MFMAs that do not depend on them.  Every
 // output element is still folded once per K group, in K order.
-template <int BN, int STAGES, int CUR, int J, bool KTAIL>
+template <int BN, int STAGES, int CUR, int J, bool KTAIL, bool TWO>
 __device__ __forceinline__ void k_step(uint4* ring, v4f (&acc)[BN / 32][J], StepHead<BN, J>& h, const DmaSources& src,
                                        int64_t kb, int64_t KB, int64_t as_sk, int64_t ws_sk, int wave, int wm,
                                        int wn, int r, int g) {
@@ -234,7 +237,7 @@ __device__ __forceinline__ void k_step(uint4* ring, v4f (&acc)[BN / 32][J], Step
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     sa[j] = h.as_v[j] * h.wa;
-    sb[j] = BN == 160 ? h.as_v[j] * h.wb : sa[j];
+    sb[j] = TWO ? h.as_v[j] * h.wb : sa[j];
   }
   v8i a[NI];
   a[0] = h.a0;
@@ -244,7 +247,7 @@ __device__ __forceinline__ void k_step(uint4* ring, v4f (&acc)[BN / 32][J], Step
 #pragma unroll
     for (int j = 0; j < J; ++j) p[i][j] = mfma_16x16x128_e4m3(a[i], h.b[j]);
     a[i + 1] = read_a<BN, CUR, J>(ring, i + 1, wn, r, g);
-    if (i > 0) fold_tile<BN, J>(acc, p[i - 1], sa, sb, src.use_b, i - 1);
+    if (i > 0) fold_tile<BN, J, TWO>(acc, p[i - 1], sa, sb, src.use_b, i - 1);
   }
 #pragma unroll
   for (int i = NA + 1; i < NI; ++i) a[i] = read_a<BN, CUR, J>(ring, i, wn, r, g);
@@ -277,10 +280,10 @@ __device__ __forceinline__ void k_step(uint4* ring, v4f (&acc)[BN / 32][J], Step
     p[i][j] = mfma_16x16x128_e4m3(a[i], h.b[j]);
 #pragma unroll
     for (int d = t * ND / NM; d < (t + 1) * ND / NM; ++d) issue_one<BN, CUR, J, KTAIL>(ring, src, ahead, KB, as_sk, wave, d);
-    if (j == J - 1 && i > 0) fold_tile<BN, J>(acc, p[i - 1], sa, sb, src.use_b, i - 1);
+    if (j == J - 1 && i > 0) fold_tile<BN, J, TWO>(acc, p[i - 1], sa, sb, src.use_b, i - 1);
     __builtin_amdgcn_sched_barrier(0);
   }
-  fold_tile<BN, J>(acc, p[NI - 1], sa, sb, src.use_b, NI - 1);
+  fold_tile<BN, J, TWO>(acc, p[NI - 1], sa, sb, src.use_b, NI - 1);
   __builtin_amdgcn_sched_barrier(0);
   h = nh;
 }
@@ -322,7 +325,7 @@ __device__ __forceinline__ void read_scales(const uint4* ring, StepRegs<BN, J>& 
 // before the last barrier, is refilled with K group kb + STAGES.  Both go out between the
 // MFMAs, and the fold of a 16x16 tile two MFMAs after its own, so neither the LDS reads nor
 // the MFMA latency stand in the chain.
-template <int BN, int STAGES, int CUR, int J, bool KTAIL>
+template <int BN, int STAGES, int CUR, int J, bool KTAIL, bool TWO>
 __device__ __forceinline__ void reg_step(uint4* ring, v4f (&acc)[BN / 32][J], const StepRegs<BN, J>& f,
                                          StepRegs<BN, J>& nf, const DmaSources& src, int64_t kb, int64_t KB,
                                          int64_t as_sk, int64_t ws_sk, int wave, int wm, int wn, int r, int g) {
@@ -335,14 +338,14 @@ __device__ __forceinline__ void reg_step(uint4* ring, v4f (&acc)[BN / 32][J], co
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     sa[j] = f.as_v[j] * f.wa;
-    sb[j] = BN == 160 ? f.as_v[j] * f.wb : sa[j];
+    sb[j] = TWO ? f.as_v[j] * f.wb : sa[j];
   }
   read_scales<BN, NXT, J>(ring, nf, src, nkb, ws_sk, wm, r);
   constexpr int kLag = 2;
   v4f p[kLag + 1];
   auto fold = [&](int t) {
     const int i = t / J, j = t % J;
-    const float sc = (BN == 160 && ((src.use_b >> i) & 1)) ? sb[j] : sa[j];
+    const float sc = (TWO && ((src.use_b >> i) & 1)) ? sb[j] : sa[j];
 #pragma unroll
     for (int v = 0; v < 4; ++v) acc[i][j][v] = __builtin_fmaf(p[t % (kLag + 1)][v], sc, acc[i][j][v]);
   };
@@ -367,7 +370,7 @@ __device__ __forceinline__ void reg_step(uint4* ring, v4f (&acc)[BN / 32][J], co
   asm volatile("" ::: "memory");
 }
 
-template <int STAGES, int BN, typename OutT, int J, bool KTAIL>
+template <int STAGES, int BN, typename OutT, int J, bool KTAIL, bool SILU>
 __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dma_kernel(
     const uint8_t* __restrict__ q, int64_t ldq, const float* __restrict__ as, int64_t as_sk,
     const uint8_t* __restrict__ w, int64_t ldw, const float* __restrict__ ws, int64_t ws_sn,
@@ -385,8 +388,13 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
   tile_of_dma(blockIdx.x, tiles_m, tiles_n, &tm, &tn);
   using G = DmaGeo<BN, J>;
   constexpr int NI = G::kNI;
+  // A wave's columns lie in one 128-column weight-scale block unless BN = 160, or the up half
+  // starts inside one.
+  constexpr bool kTwo = BN == 160 || SILU;
   const int64_t m0 = tm * G::kRows;
-  const int64_t n0 = tn * BN;
+  // SILU: the tile's first BN / 2 weight rows are gate rows n0 .., the rest up rows N / 2 + n0 ...
+  const int64_t half = N / 2;
+  const int64_t n0 = tn * (SILU ? BN / 2 : BN);
 
   DmaSources src;
   src.w = w + n0 * ldw;
@@ -396,7 +404,11 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
   for (int i = 0; i < 5; ++i) {
     const int rr = (i * 4 + wave) * 8 + (lane >> 3);
     const int c = (lane & 7) ^ (rr & 7);
-    const int64_t wrow = (n0 + rr) < N ? rr : (N - 1 - n0);
+    int64_t wrow = (n0 + rr) < N ? rr : (N - 1 - n0);
+    if (SILU) {
+      const int64_t hr = rr < BN / 2 ? rr : rr - BN / 2;
+      wrow = (n0 + hr < half ? hr : half - 1 - n0) + (rr < BN / 2 ? 0 : half);
+    }
     src.woff[i] = static_cast<uint32_t>(wrow * ldw + 16 * c);
     // Chunks of the last group past K read the group's first chunk of the same row: the
     // activation codes there are zero, and a NaN code can only come from the row itself.
@@ -414,7 +426,7 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
   }
   {
     // The wave's columns [nw, nw + BN/2) touch at most two 128-column weight-scale blocks.
-    const int64_t nw = n0 + wn * (BN / 2);
+    const int64_t nw = n0 + wn * (SILU ? half : BN / 2);
     const int64_t last_blk = (N - 1) / kGroup;
     const int64_t blk_a = nw / kGroup < last_blk ? nw / kGroup : last_blk;
     const int64_t blk_b = blk_a + 1 < last_blk ? blk_a + 1 : last_blk;
@@ -447,7 +459,7 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
   if constexpr (STAGES == 2) {
     StepHead<BN, J> h;
     read_head<BN, 0, J>(ring, h, src, 0, ws_sk, wm, wn, r, g);
-#define MI355X_KSTEP(S, KBV) k_step<BN, STAGES, S, J, KTAIL>(ring, acc, h, src, KBV, KB, as_sk, ws_sk, wave, wm, wn, r, g)
+#define MI355X_KSTEP(S, KBV) k_step<BN, STAGES, S, J, KTAIL, kTwo>(ring, acc, h, src, KBV, KB, as_sk, ws_sk, wave, wm, wn, r, g)
     for (; kb + 2 <= KB; kb += 2) {
       MI355X_KSTEP(0, kb);
       MI355X_KSTEP(1, kb + 1);
@@ -463,7 +475,7 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #define MI355X_KSTEP(S, F, NF, KBV) \
-  reg_step<BN, STAGES, S, J, KTAIL>(ring, acc, F, NF, src, KBV, KB, as_sk, ws_sk, wave, wm, wn, r, g)
+  reg_step<BN, STAGES, S, J, KTAIL, kTwo>(ring, acc, F, NF, src, KBV, KB, as_sk, ws_sk, wave, wm, wn, r, g)
     for (; kb + STAGES <= KB; kb += STAGES) {
       MI355X_KSTEP(0, f0, f1, kb);
       MI355X_KSTEP(1, f1, f0, kb + 1);
@@ -499,24 +511,18 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
       }
     }
     __syncthreads();
-    constexpr int C = BN / 8;  // 16-byte pieces per row
-    static_assert((G::kRows * C) % kDmaThreads == 0, "whole passes");
+    constexpr int C = (SILU ? BN / 2 : BN) / 8;  // 16-byte pieces per row
+    static_assert((G::kRows * BN / 8) % kDmaThreads == 0, "whole passes");
+    const int64_t n_end = SILU ? half : N;
 #pragma unroll
-    for (int it = 0; it < G::kRows * C / kDmaThreads; ++it) {
-      const int idx = tid + it * kDmaThreads;
+    for (int idx = tid; idx < G::kRows * C; idx += kDmaThreads) {
       const int row = idx / C, c = idx - (idx / C) * C;
       const int64_t m = m0 + row, n = n0 + 8 * c;
       const uint16_t* reg_r = reinterpret_cast<const uint16_t*>(row < kHalf ? stage0 : stage1);
-      const uint4 val = *reinterpret_cast<const uint4*>(reg_r + staged_index<BN>(row % kHalf, 8 * c));
-      if (m >= M) continue;
-      uint16_t* dst = out + m * ldo + n;
-      if (n + 8 <= N) {
-        store16_nt(dst, val);
-      } else {
-        const uint16_t* hv = reinterpret_cast<const uint16_t*>(&val);
-        for (int v = 0; v < 8; ++v)
-          if (n + v < N) dst[v] = hv[v];
-      }
+      uint4 val = *reinterpret_cast<const uint4*>(reg_r + staged_index<BN>(row % kHalf, 8 * c));
+      if constexpr (SILU)
+        val = silu_mul8(val, *reinterpret_cast<const uint4*>(reg_r + staged_index<BN>(row % kHalf, BN / 2 + 8 * c)));
+      if (m < M) store8_cols(out + m * ldo + n, val, n, n_end);
     }
     return;
   }
@@ -559,7 +565,7 @@ bool tile_dma_supported(const uint8_t* q, int64_t ldq, int64_t as_sm, int64_t as
 
 int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_sk, const uint8_t* w,
                     int64_t ldw, const float* ws, int64_t ws_sn, int64_t ws_sk, void* out, int out_dtype,
-                    int64_t ldo, int64_t M, int64_t N, int64_t K, int bn, int rows, hipStream_t stream) {
+                    int64_t ldo, int64_t M, int64_t N, int64_t K, int bn, int rows, hipStream_t stream, bool silu) {
   if (bn != 64 && bn != 128 && bn != 160) return MI355X_FP8_ERR_INVALID;
   if (rows != 128 && ((rows != 64 && rows != 96) || bn == 160)) return MI355X_FP8_ERR_INVALID;
   const int64_t tiles_m = (M + rows - 1) / rows;
@@ -569,17 +575,20 @@ int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_s
   dim3 grid(static_cast<unsigned>(tiles_m * tiles_n));
   const int tail = static_cast<int>(K % kGroup);
   uint16_t* o = static_cast<uint16_t*>(out);
+  if (silu && (vec_out != 2 || out_dtype != kBF16 || tail != 0)) return MI355X_FP8_ERR_INVALID;
   // Two stages (76 KiB, room for the 160-wide W tile) let two workgroups share a CU.  When the
   // tiles do not fill the CUs anyway, four stages (one workgroup per CU) keep more K groups in
   // flight; six, where they fit, measured the same (28.0 and 28.3 us for N = 2560, K = 9728 at
   // 536 rows).  64x64 tiles have room for two workgroups of four stages.
   const bool few = tiles_m * tiles_n <= device_cus();
 #define MI355X_DMA_ARGS q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, o, ldo, M, N, (K + kGroup - 1) / kGroup, tiles_m, tiles_n, vec_out, tail
-#define MI355X_DMA_LAUNCH_K(ST, BN, J, KT)                                                                            \
-  (out_dtype == kBF16 ? tile_gemm_dma_kernel<ST, BN, bf16_t, J, KT><<<grid, kDmaThreads, 0, stream>>>(MI355X_DMA_ARGS) \
-                      : tile_gemm_dma_kernel<ST, BN, f16_t, J, KT><<<grid, kDmaThreads, 0, stream>>>(MI355X_DMA_ARGS))
-#define MI355X_DMA_LAUNCH(ST, BN, J) \
-  (tail == 0 ? MI355X_DMA_LAUNCH_K(ST, BN, J, false) : MI355X_DMA_LAUNCH_K(ST, BN, J, true))
+#define MI355X_DMA_LAUNCH_T(ST, BN, T, J, KT, SI) \
+  tile_gemm_dma_kernel<ST, BN, T, J, KT, SI><<<grid, kDmaThreads, 0, stream>>>(MI355X_DMA_ARGS)
+#define MI355X_DMA_LAUNCH_K(ST, BN, J, KT)                                       \
+  (out_dtype == kBF16 ? MI355X_DMA_LAUNCH_T(ST, BN, bf16_t, J, KT, false) : MI355X_DMA_LAUNCH_T(ST, BN, f16_t, J, KT, false))
+#define MI355X_DMA_LAUNCH(ST, BN, J)                            \
+  (silu ? MI355X_DMA_LAUNCH_T(ST, BN, bf16_t, J, false, true)   \
+        : tail == 0 ? MI355X_DMA_LAUNCH_K(ST, BN, J, false) : MI355X_DMA_LAUNCH_K(ST, BN, J, true))
 #define MI355X_DMA_ROWS(BN, J)                              \
   do {                                                      \
     if (few) MI355X_DMA_LAUNCH(kStagesFew, BN, J);          \
@@ -600,6 +609,7 @@ int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_s
 #undef MI355X_DMA_ROWS
 #undef MI355X_DMA_LAUNCH
 #undef MI355X_DMA_LAUNCH_K
+#undef MI355X_DMA_LAUNCH_T
 #undef MI355X_DMA_ARGS
   return hipGetLastError() == hipSuccess ? MI355X_FP8_OK : MI355X_FP8_ERR_LAUNCH;
 }

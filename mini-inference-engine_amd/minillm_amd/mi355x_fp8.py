@@ -313,6 +313,35 @@ def launch_block_gemm(activation: torch.Tensor, weight: torch.Tensor, output: to
         None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), code, stream))
 
 
+def _gemm_silu_takes(m: int, k: int, weight: torch.Tensor, scales: torch.Tensor, device: torch.device) -> bool:
+    """Whether a call may go to ``_gemm_silu``: the facts the C-ABI cannot see (as
+    ``_check_gemm_operands`` raises for), more than 16 rows and whole K groups.  Other calls take
+    the separate GEMM and SiLU*up, which raise what they raise."""
+
+    return bool(
+        m > 16 and k % 128 == 0 and weight.ndim == 2 and scales.ndim == 2 and weight.shape[0] % 32 == 0
+        and weight.shape[1] == k and weight.dtype == torch.float8_e4m3fn and scales.dtype == torch.float32
+        and weight.stride(1) == 1 and weight.stride(0) >= k and weight.device == scales.device == device
+        and tuple(scales.shape) == (-(-weight.shape[0] // 128), k // 128)
+    )
+
+
+def _gemm_silu(q: torch.Tensor, s: torch.Tensor, weight: torch.Tensor, scales: torch.Tensor) -> torch.Tensor | None:
+    """h = silu(gate) * up [M, N / 2] (bf16) of the merged gate/up GEMM on quantized activations,
+    in the prefill kernels' epilogue, or None (nothing launched) where those do not take it."""
+
+    m, k = q.shape
+    n = int(weight.shape[0])
+    h = torch.empty((m, n // 2), device=q.device, dtype=torch.bfloat16)
+    code = _lib.load().mi355x_fp8_block_gemm_silu(
+        q.data_ptr(), q.stride(0), s.data_ptr(), s.stride(0), s.stride(1), weight.data_ptr(), weight.stride(0),
+        scales.data_ptr(), scales.stride(0), scales.stride(1), h.data_ptr(), h.stride(0), m, n, k, _stream_ptr(q.device))
+    if code == _lib.ERR_UNSUPPORTED:
+        return None
+    _lib.check(code)
+    return h
+
+
 def mi355x_fp8_linear(
     input: torch.Tensor,
     weight: torch.Tensor,
@@ -644,8 +673,9 @@ def rmsnorm_gate_up_silu_mi355x_fp8(x: torch.Tensor, norm_weight: torch.Tensor, 
     given.
 
     Up to 8 rows (bf16, K a multiple of 256 up to 2560) the three run as one launch, each
-    workgroup owning matching gate and up weight rows; otherwise the norm-linear and the
-    SiLU*up kernel run separately.  Both give the same bits: h = bf16(bf16(silu(g)) * u) on the
+    workgroup owning matching gate and up weight rows; at prefill sizes the GEMM applies SiLU*up in
+    its epilogue, behind the norm-quantizer; otherwise the norm-linear and the SiLU*up kernel run
+    separately.  All give the same bits: h = bf16(bf16(silu(g)) * u) on the
     projection's bf16 gate and up outputs, as ``silu_mul_quant_mi355x_fp8`` forms it."""
 
     k = int(x.shape[-1])
@@ -677,6 +707,17 @@ def rmsnorm_gate_up_silu_mi355x_fp8(x: torch.Tensor, norm_weight: torch.Tensor, 
             h = h.reshape(*x.shape[:-1], inter)
             return (h, summed.reshape(x.shape)) if residual is not None else h
 
+    if _gemm_silu_takes(x2.shape[0], k, gate_up_weight, gate_up_scale, x.device):
+        outs = rmsnorm_quant_mi355x_fp8(x, norm_weight, eps, residual)
+        q, s = outs[0].reshape(-1, k), outs[1]
+        h = _gemm_silu(q, s, gate_up_weight, gate_up_scale)
+        if h is None:
+            gu2 = torch.empty((q.shape[0], n), device=x.device, dtype=torch.bfloat16)
+            launch_block_gemm(q, gate_up_weight, gu2, s, gate_up_scale)
+            h = silu_mul_quant_mi355x_fp8(gu2[:, :inter], gu2[:, inter:], return_intermediate=True)[0]
+        h = h.reshape(*x.shape[:-1], inter)
+        return (h, outs[2]) if residual is not None else h
+
     outs = rmsnorm_linear_mi355x_fp8(x, norm_weight, eps, gate_up_weight, gate_up_scale, residual)
     gu = outs[0] if residual is not None else outs
     gu2 = gu.reshape(-1, n)
@@ -691,16 +732,26 @@ def mlp_forward_mi355x_fp8(x: torch.Tensor, gate_up_weight: torch.Tensor, gate_u
     """Qwen3 MLP on FP8 weights: ``down(SiLU(gate) * up)`` with merged gate/up.
 
     The reference's _mlp_forward (engine/kernels/fused.py:280-283) runs merged gate_up ->
-    silu_mul -> down_proj, quantizing the bf16 product again inside down_proj.  Here the
-    SiLU-mul writes the quantized product directly (one kernel instead of silu_mul plus the
-    down projection's quantizer); the codes are those the quantizer would give for the
-    same bf16 product.
+    silu_mul -> down_proj, quantizing the bf16 product again inside down_proj.  Here, at prefill
+    sizes, the gate/up GEMM's epilogue forms the bf16 product and the quantizer reads that;
+    elsewhere the SiLU-mul writes the quantized product directly (one kernel instead of silu_mul
+    plus the down projection's quantizer).  The codes are those the quantizer would give for the
+    same bf16 product either way.
     """
 
     k = int(x.shape[-1])
-    gate_up = mi355x_fp8_linear(x.reshape(-1, k), gate_up_weight, gate_up_scale, [128, 128])
-    inter = gate_up.shape[-1] // 2
-    q, s = silu_mul_quant_mi355x_fp8(gate_up[:, :inter], gate_up[:, inter:])
+    x2 = x.reshape(-1, k)
+    h = None
+    if (x.dtype == torch.bfloat16 and _supports_call(x2, gate_up_weight, gate_up_scale, SUPPORTED_BLOCK_SIZE, None)
+            and _gemm_silu_takes(x2.shape[0], k, gate_up_weight, gate_up_scale, x.device)):
+        q, s = quantize_mi355x_fp8_activation(x2, scale_layout="kgroup")
+        h = _gemm_silu(q, s, gate_up_weight, gate_up_scale)
+    if h is not None:
+        q, s = quantize_mi355x_fp8_activation(h, scale_layout="kgroup")
+    else:
+        gate_up = mi355x_fp8_linear(x2, gate_up_weight, gate_up_scale, [128, 128])
+        inter = gate_up.shape[-1] // 2
+        q, s = silu_mul_quant_mi355x_fp8(gate_up[:, :inter], gate_up[:, inter:])
     out = torch.empty((q.shape[0], down_weight.shape[0]), device=x.device, dtype=output_dtype or x.dtype)
     if q.shape[0]:
         launch_block_gemm(q, down_weight if down_weight.stride(-1) == 1 else down_weight.contiguous(), out, s,

@@ -58,3 +58,46 @@ def test_k_tail_keeps_a_nan_code_in_its_own_column(k):
     assert torch.isnan(got).all(dim=0).nonzero().flatten().tolist() == [5, 17]
     keep = [c for c in range(n) if c not in (5, 17)]
     assert bitwise_equal(got[:, keep], ref[:, keep])
+
+
+@pytest.mark.parametrize("m,inter,k", [
+    # The Qwen3-4B width at row counts that pick each tile shape; halves that end inside a tile or
+    # inside a weight-scale block; one K group.
+    (17, 9728, 256), (100, 9728, 128), (160, 9728, 384), (300, 9728, 256), (512, 9728, 256), (536, 9728, 640),
+    (864, 9728, 128), (1024, 9728, 256), (2048, 9728, 384), (2208, 9728, 256), (200, 1040, 256), (333, 3008, 384),
+    (1000, 1616, 128), (65, 16, 256), (2500, 4880, 256),
+])
+def test_silu_epilogue_equals_gemm_then_silu(m, inter, k):
+    """h of the gate/up GEMM's epilogue against the GEMM followed by the SiLU*up kernel, bit for
+    bit, and through the two public calls that use it."""
+
+    x = make_activations(m, k, 3).cuda()
+    w, ws = make_weights(ModelShape("gate_up", 2 * inter, k), 3, "cuda")
+    q, s = fp8.quantize_mi355x_fp8_activation(x, scale_layout="kgroup")
+    gate_up = torch.empty((m, 2 * inter), device="cuda", dtype=torch.bfloat16)
+    fp8.launch_block_gemm(q, w, gate_up, s, ws)
+    ref = fp8.silu_mul_quant_mi355x_fp8(gate_up[:, :inter], gate_up[:, inter:], return_intermediate=True)[0]
+    h = fp8._gemm_silu(q, s, w, ws)
+    if h is None:  # the decode kernel takes these rows
+        assert fp8.dispatch_name(m, 2 * inter, k).startswith("stream")
+    else:
+        assert bitwise_equal(h, ref), bit_mismatch_details(h, ref)
+    down, down_s = make_weights(ModelShape("down", 256, inter), 5, "cuda")
+    out = fp8.mlp_forward_mi355x_fp8(x, w, ws, down, down_s)
+    expect = torch.empty((m, 256), device="cuda", dtype=torch.bfloat16)
+    hq, hs = fp8.quantize_mi355x_fp8_activation(ref, scale_layout="kgroup")
+    fp8.launch_block_gemm(hq, down, expect, hs, down_s)
+    assert bitwise_equal(out, expect), bit_mismatch_details(out, expect)
+
+
+def test_silu_epilogue_refuses_what_it_cannot_take():
+    """Decode rows, K inside a group, an odd number of 16-column tiles and row-major scales go to the
+    separate kernels."""
+
+    k = 256
+    w, ws = make_weights(ModelShape("gate_up", 512, k), 1, "cuda")
+    assert not fp8._gemm_silu_takes(16, k, w, ws, w.device)
+    assert not fp8._gemm_silu_takes(200, k, w[:496], ws, w.device)
+    assert not fp8._gemm_silu_takes(200, 240, w[:, :240], ws, w.device)
+    q, s = fp8.quantize_mi355x_fp8_activation(make_activations(200, k, 1).cuda())
+    assert fp8._gemm_silu(q, s, w, ws) is None
