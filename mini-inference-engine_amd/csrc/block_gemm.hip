@@ -601,9 +601,10 @@ __global__ __launch_bounds__(kStreamWaves * 64) void stream_gemm_kernel(
       // bf16 output, then silu = bf16(g / (1 + exp(-g))) and h = bf16(silu * u): the
       // arithmetic of silu_mul_quant_kernel on the bf16 gate/up outputs.
       const float* sfu = scl + (2 + ((n_rows + n0 + nl) / kGroup != nbu0 ? 1 : 0)) * kTokS + tok;
-      const float g = bf16_bits_val(OutCvt<bf16_t>::cvt(fold(pf, sf)));
+      float g[1] = {bf16_bits_val(OutCvt<bf16_t>::cvt(fold(pf, sf)))};
       const float u = bf16_bits_val(OutCvt<bf16_t>::cvt(fold(pf + 16 * kHalfT, sfu)));
-      out[(m_base + tok) * ldo + n0 + nl] = silu_mul_bf16(g, u);
+      silu_bf16(g);
+      out[(m_base + tok) * ldo + n0 + nl] = f32_to_bf16_bits(g[0] * u);
     } else {
       const float acc = fold(pf, sf);
       if (RAGGED || n0 + nl < N) out[(m_base + tok) * ldo + n0 + nl] = OutCvt<OutT>::cvt(acc);

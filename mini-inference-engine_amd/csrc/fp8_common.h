@@ -79,19 +79,45 @@ __device__ __forceinline__ float round_bf16(float f) {
   return __uint_as_float(static_cast<uint32_t>(f32_to_bf16_bits(f)) << 16);
 }
 
-// The reference's silu_mul on bf16 gate and up values (engine/kernels/fused.py:127-137):
-// silu = bf16(g / (1 + exp(-g))), then the bf16 product's bits.
-__device__ __forceinline__ uint16_t silu_mul_bf16(float g, float u) {
-  return f32_to_bf16_bits(round_bf16(g / (1.0f + expf(-g))) * u);
+// bf16(g / (1 + exp(-g))) of N bf16 gate values, in place.  The function depends on the 16 bits of
+// g alone, so the short form below (the hardware exp2 and reciprocal, one Newton step on the
+// reciprocal) was compared with the IEEE division and expf over all 65536 of them: equal bits
+// wherever g > -86.  Below that, where 1 + exp(-g) nears the largest float and its reciprocal the
+// denormals, and for a NaN, the group takes the long form.  About 13 issue slots an element
+// instead of 32: the SiLU*up quantizer at 2048 x 9728 33.4 -> 25.8 us.
+template <int N>
+__device__ __forceinline__ void silu_bf16(float (&g)[N]) {
+  bool fast = true;
+#pragma unroll
+  for (int i = 0; i < N; ++i) fast &= g[i] > -86.0f;
+  if (fast) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const float d = 1.0f + __builtin_amdgcn_exp2f(g[i] * -1.44269504088896341f);
+      const float r = __builtin_amdgcn_rcpf(d);
+      g[i] = round_bf16(g[i] * __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r));
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) g[i] = round_bf16(g[i] / (1.0f + expf(-g[i])));
+  }
 }
-// Eight of them: two 16-byte pieces of gate and up columns in, one of h out.
+// The reference's silu_mul (engine/kernels/fused.py:127-137) on eight columns: two 16-byte pieces of
+// bf16 gate and up values in, the bf16 products out.
 __device__ __forceinline__ uint4 silu_mul8(uint4 gate, uint4 up) {
   const uint32_t gw[4] = {gate.x, gate.y, gate.z, gate.w}, uw[4] = {up.x, up.y, up.z, up.w};
+  float g[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    g[2 * i] = __uint_as_float(gw[i] << 16);
+    g[2 * i + 1] = __uint_as_float(gw[i] & 0xffff0000u);
+  }
+  silu_bf16(g);
   uint32_t h[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    h[i] = silu_mul_bf16(__uint_as_float(gw[i] << 16), __uint_as_float(uw[i] << 16)) |
-           (static_cast<uint32_t>(silu_mul_bf16(__uint_as_float(gw[i] & 0xffff0000u), __uint_as_float(uw[i] & 0xffff0000u))) << 16);
+    h[i] = f32_to_bf16_bits(g[2 * i] * __uint_as_float(uw[i] << 16)) |
+           (static_cast<uint32_t>(f32_to_bf16_bits(g[2 * i + 1] * __uint_as_float(uw[i] & 0xffff0000u))) << 16);
   return make_uint4(h[0], h[1], h[2], h[3]);
 }
 // Stores 8 consecutive 16-bit values at dst, columns [n, n + 8) of end.

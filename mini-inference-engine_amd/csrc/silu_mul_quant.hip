@@ -5,7 +5,7 @@
 //   silu = bf16( g / (1 + exp(-g)) )      fp32 math, IEEE division
 //   h    = bf16( silu * u )               fp32 product of two bf16 values
 // and the quantizer is exactly act_quant.hip's (engine/kernels/sm89_fp8.py:304-332) applied
-// to h.  exp() is ROCm's expf (faithfully rounded); the reference's CUDA exp may differ in
+// to h.  exp() has ROCm's expf bits (silu_bf16); the reference's CUDA exp may differ in
 // the last place, which can move h by one bf16 ulp: the quantized codes and scales are
 // bit-exact with respect to this kernel's own h, which it can also write out.
 //
@@ -56,9 +56,10 @@ __global__ __launch_bounds__(kSmqThreads) void silu_mul_quant_kernel(
 
   float t[8];
   uint16_t hb[8];
+  silu_bf16(gv);
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    hb[i] = silu_mul_bf16(gv[i], uv[i]);
+    hb[i] = f32_to_bf16_bits(gv[i] * uv[i]);
     t[i] = __uint_as_float(static_cast<uint32_t>(hb[i]) << 16);
   }
   uint32_t packed[2];

@@ -101,3 +101,24 @@ def test_silu_epilogue_refuses_what_it_cannot_take():
     assert not fp8._gemm_silu_takes(200, 240, w[:, :240], ws, w.device)
     q, s = fp8.quantize_mi355x_fp8_activation(make_activations(200, k, 1).cuda())
     assert fp8._gemm_silu(q, s, w, ws) is None
+
+
+def test_silu_over_every_bf16_gate():
+    """silu(g) for all 65536 bf16 gates (up = 1): the short form within half a bf16 place of the
+    exact value plus its own fp32 error (below 2^-20, so 2^-10 of the half place is ample); the
+    separate kernel and the GEMM epilogue's form share it.  Infinities, NaN and gates whose
+    exponential overflows keep the long form's values."""
+
+    gate = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).cuda().view(512, 128)
+    h = fp8.silu_mul_quant_mi355x_fp8(gate, torch.ones_like(gate), return_intermediate=True)[0]
+    g64, h64 = gate.double().cpu().flatten(), h.double().cpu().flatten()
+    exact = g64 / (1 + torch.exp(-g64))
+    inside = torch.isfinite(g64) & (g64 > -80) & (exact.abs() > 2.0 ** -120)
+    half_place = torch.exp2(torch.floor(torch.log2(exact[inside].abs()))) * 2.0 ** -8
+    assert ((h64[inside] - exact[inside]).abs() <= half_place * (1 + 2.0 ** -10)).all()
+    assert h64[g64 == float("inf")].item() == float("inf")
+    assert torch.isnan(h64[torch.isnan(g64)]).all() and torch.isnan(h64[g64 == -float("inf")]).all()
+    deep = torch.isfinite(g64) & (g64 < -89)
+    assert (h64[deep] == 0).all() and torch.signbit(h64[deep]).all()
+    zero = h.flatten()[gate.flatten() == 0].cpu()
+    assert torch.signbit(zero).tolist() == torch.signbit(gate.flatten()[gate.flatten() == 0].cpu()).tolist()
