@@ -180,8 +180,13 @@ struct Scales {
 // sixteen partials are folded while they run (one MFMA per four FMAs), so no fold waits on
 // the MFMA it follows.  The eight scale products a_s[j] * w_s (two weight-scale blocks at
 // most) are formed once per step; each is the same single fp32 product as before, so the
-// folded values are unchanged bit for bit.
-template <int BN, int J, int NS, int S, int NXT>
+// folded values are unchanged bit for bit.  Where a wave's columns always lie in one block
+// (TWO = false: widths 256 and 128) no tile selects between the two sets: 40 of the 256-wide
+// step's 190 VALU instructions went, and the kernel is bound by its issue slots as much as by its
+// feed (N = 19456, K = 2560 at 4096 rows 201.7 -> 198.4 us, 192x256 at 536 rows 38.8 -> 37.5).
+// Folding two or three MFMAs behind instead of a whole column tile, in fewer registers, measured
+// the same or slower (201.7 -> 199.5-203 at 256 wide, 112 -> 113 at 224).
+template <int BN, int J, int NS, int S, int NXT, bool TWO>
 __device__ __forceinline__ void compute256(v4f (&acc)[BN / 32][J], const Scales& sc_in, uint32_t use_b, int wm,
                                            int wn, int r, int g, const Src256& src, const uint8_t* w,
                                            const uint8_t* q, int64_t kn, int wave) {
@@ -194,7 +199,7 @@ __device__ __forceinline__ void compute256(v4f (&acc)[BN / 32][J], const Scales&
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     sa[j] = sc_in.a[j] * sc_in.wa;
-    sb[j] = sc_in.a[j] * sc_in.wb;
+    sb[j] = TWO ? sc_in.a[j] * sc_in.wb : sa[j];
   }
   v8i a0 = frag<S>(st, wrow0, g);
   v8i b[J];
@@ -213,7 +218,7 @@ __device__ __forceinline__ void compute256(v4f (&acc)[BN / 32][J], const Scales&
     }
     // MFMA (i, j), then the fold of (i - 1, j), whose MFMA went out four MFMAs earlier; the
     // scheduling barriers keep that order, so no fold waits on the MFMA just issued.
-    const bool ub = i > 0 && ((use_b >> (i - 1)) & 1);
+    const bool ub = TWO && i > 0 && ((use_b >> (i - 1)) & 1);
 #pragma unroll
     for (int j = 0; j < J; ++j) {
       if (i < NI) p[i & 1][j] = mfma_16x16x128_e4m3(a0, b[j]);
@@ -234,7 +239,7 @@ __device__ __forceinline__ void compute256(v4f (&acc)[BN / 32][J], const Scales&
 
 // The unpipelined fold, for the 256-row, 256-wide tiles: their accumulators leave no registers
 // for a second set of partials (the pipelined form spills there; the 192-row form has room).
-template <int BN, int J, int NS, int S, int NXT>
+template <int BN, int J, int NS, int S, int NXT, bool TWO>
 __device__ __forceinline__ void compute256_plain(v4f (&acc)[BN / 32][J], const Scales& sc_in, uint32_t use_b,
                                                  int wm, int wn, int r, int g, const Src256& src, const uint8_t* w,
                                                  const uint8_t* q, int64_t kn, int wave) {
@@ -243,6 +248,12 @@ __device__ __forceinline__ void compute256_plain(v4f (&acc)[BN / 32][J], const S
   constexpr int NDMA = G::kNDma;
   const uint4* st = stage256<NS, S>();
   const int wrow0 = wn * (BN / 2) + r;
+  float sa[J], sb[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    sa[j] = sc_in.a[j] * sc_in.wa;
+    sb[j] = TWO ? sc_in.a[j] * sc_in.wb : sa[j];
+  }
   v8i a0 = frag<S>(st, wrow0, g);
   v8i b[J];
 #pragma unroll
@@ -255,13 +266,13 @@ __device__ __forceinline__ void compute256_plain(v4f (&acc)[BN / 32][J], const S
       if ((t < NDMA / 2 ? 0 : NI / 2) == i) issue_one<BN, J, NS, NXT>(src, w, q, kn, wave, t);
     v8i a2;
     if (i + 2 < NI) a2 = frag<S>(st, wrow0 + 16 * (i + 2), g);
-    const float wsv = (use_b >> i) & 1 ? sc_in.wb : sc_in.wa;
+    const bool ub = TWO && ((use_b >> i) & 1);
     v4f p[J];
 #pragma unroll
     for (int j = 0; j < J; ++j) p[j] = mfma_16x16x128_e4m3(a0, b[j]);
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-      const float sc = sc_in.a[j] * wsv;
+      const float sc = ub ? sb[j] : sa[j];
 #pragma unroll
       for (int v = 0; v < 4; ++v) acc[i][j][v] = __builtin_fmaf(p[j][v], sc, acc[i][j][v]);
     }
@@ -297,7 +308,7 @@ __device__ __forceinline__ void load_scales(Scales& s, const Src256& src, int64_
 // ahead (the one read in the previous step); the end-of-step wait leaves only that newest
 // batch in flight (loads complete in issue order).  Past the end of the range the loads
 // repeat its last group (the stage they fill is not read again).
-template <int BN, int J, int NS, int CUR>
+template <int BN, int J, int NS, int CUR, bool TWO>
 __device__ __forceinline__ void step256(v4f (&acc)[BN / 32][J], const Scales& cur, Scales& next,
                                         const Src256& src, const uint8_t* w, const uint8_t* q, int64_t kb,
                                         int64_t khi, int64_t as_sk, int64_t ws_sk, int wave, int wm, int wn, int r,
@@ -310,9 +321,9 @@ __device__ __forceinline__ void step256(v4f (&acc)[BN / 32][J], const Scales& cu
   asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (BN == 256 && J == 4)
-    compute256_plain<BN, J, NS, CUR, (CUR + NS - 1) % NS>(acc, cur, src.use_b, wm, wn, r, g, src, w, q, kd, wave);
+    compute256_plain<BN, J, NS, CUR, (CUR + NS - 1) % NS, TWO>(acc, cur, src.use_b, wm, wn, r, g, src, w, q, kd, wave);
   else
-    compute256<BN, J, NS, CUR, (CUR + NS - 1) % NS>(acc, cur, src.use_b, wm, wn, r, g, src, w, q, kd, wave);
+    compute256<BN, J, NS, CUR, (CUR + NS - 1) % NS, TWO>(acc, cur, src.use_b, wm, wn, r, g, src, w, q, kd, wave);
   // Every MFMA of the step is issued before the wait: the matrix core then works through
   // them while the wave waits for its DMA and the other waves (without this barrier the
   // scheduler moves the last MFMA groups behind s_barrier; measured 7 % slower on qkv).
@@ -393,7 +404,7 @@ __device__ __forceinline__ void setup_tile(Src256& src, const Dims256& d, int64_
 
 // acc = the tile's products over K groups [klo, khi), in increasing order, through a ring
 // of NS (2 or 3) LDS stages.
-template <int BN, int J, int NS>
+template <int BN, int J, int NS, bool TWO>
 __device__ __forceinline__ void run_k(v4f (&acc)[BN / 32][J], const Src256& src, const Dims256& d, int64_t klo,
                                       int64_t khi, int wave, int wm, int wn, int r, int g) {
   static_assert(NS == 2 || (NS == 3 && BN <= kMaxBN3), "ring depth");
@@ -403,7 +414,7 @@ __device__ __forceinline__ void run_k(v4f (&acc)[BN / 32][J], const Src256& src,
 #pragma unroll
     for (int j = 0; j < J; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 #define MI355X_STEP(CUR, SC, SN, KB) \
-  step256<BN, J, NS, CUR>(acc, SC, SN, src, d.w, d.q, KB, khi, d.as_sk, d.ws_sk, wave, wm, wn, r, g)
+  step256<BN, J, NS, CUR, TWO>(acc, SC, SN, src, d.w, d.q, KB, khi, d.as_sk, d.ws_sk, wave, wm, wn, r, g)
   if constexpr (NS == 2) {
     Scales s_even, s_odd;
     load_scales<J>(s_even, src, klo, d.as_sk, d.ws_sk);
@@ -522,7 +533,10 @@ __global__ __launch_bounds__(kT256Threads, 2) void tile256_gemm_kernel(Dims256 d
   const int64_t n0 = tn * (SILU ? BN / 2 : BN);
   setup_tile<BN, J, SILU>(src, d, tm * RT, n0, wave, lane, wm, wn, r);
   v4f acc[Geo<BN, J>::kNI][J];
-  run_k<BN, J, NS>(acc, src, d, 0, d.KB, wave, wm, wn, r, g);
+  // A wave's columns lie in one 128-column weight-scale block when BN / 2 divides 128, unless the
+  // up half starts inside one.
+  constexpr bool kTwo = SILU || 128 % (BN / 2) != 0;
+  run_k<BN, J, NS, kTwo>(acc, src, d, 0, d.KB, wave, wm, wn, r, g);
   __builtin_amdgcn_s_waitcnt(0x70);  // no DMA may still target LDS when the workgroup ends
   if (SILU || d.vec_out == 2) store_tile_lds<BN, J, NS, OutT, SILU>(acc, d, tm * RT, n0, wm, wn, r, g, tid);
   else store_tile<BN, J, OutT>(acc, d, tm * RT, n0, wm, wn, r, g);
