@@ -168,8 +168,8 @@ size_t mi355x_fp8_linear_noalloc_scratch_bytes(void);
  * kernel the automatic dispatch runs for an M x N output (M above the decode range, LDS-DMA
  * preconditions met) on a device with `cus` CUs, from the table of measured wave times:
  * *rows = tile rows (64 or 128: the LDS-DMA kernel; 192 or 256: the 256-row kernel and its
- * 192-row form), *bn = tile width.  The launch shortens a 128-row tile of width 64 or 128 to 96
- * rows when those still number at most one per CU.  Pure host computation: no device is touched.
+ * 192-row form), *bn = tile width.  An LDS-DMA tile that fits one per CU is launched as the
+ * cheapest of 64, 96 or 128 rows by 64, 96 or 128 columns that still does.  Pure host computation: no device is touched.
  */
 int mi355x_fp8_prefill_choice(int64_t M, int64_t N, int64_t cus, int* rows, int* bn);
 

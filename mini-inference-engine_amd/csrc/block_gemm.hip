@@ -851,7 +851,7 @@ int64_t device_cus() {
 // A last, partly filled wave costs 0.7 + 0.3 x its fill of a full one (a half-filled wave
 // measured 0.75-0.98).  Every kernel gives the same bits, so the choice may follow M.
 // (The figures rank the tiles; the 128-row kernel's single waves have since become 10-20 % faster
-// in the same order, and prefill_tile shortens its tiles to 96 rows where those fit.)
+// in the same order, and prefill_tile narrows its tiles where smaller ones fit one per CU.)
 namespace {
 struct TileVariant {
   int rows, bn;
@@ -897,16 +897,24 @@ PrefillChoice choose_prefill(int64_t M, int64_t N, int64_t cus, bool rows256_ok)
   return best;
 }
 
-// The tile that is launched: the model's choice, 128-row tiles in 96 rows where those still fit
-// one per CU: more CUs share the rows, and a tile's serial K loop has a quarter less to multiply
-// and a sixth less to load per step.
-// Measured 128 against 96 rows (us, weights from HBM, N = 2560): 64 wide, K = 9728 at 512
-// rows 34.1 / 26.9, at 536 27.9 / 27.6, K = 4096 at 536 12.6 / 12.2; 128 wide, K = 4096 at
-// 1024 rows 21.3 / 18.4, K = 9728 48.3 / 41.1.
+// The tile that is launched: the model's choice, and where that is a tile of the LDS-DMA kernel
+// that fits one per CU, the cheapest of these that still does (in the order of their measured
+// time over a K group: a single wave takes as long whether it fills the CUs or not, so a smaller
+// tile that spreads over more of them is free).  Measured, the model's tile against the one
+// launched (us, weights from HBM): 536 x 2560 x 4096 128x64 12.6 / 96x64 12.2; 512 x 2560 x 9728
+// 34.1 / 26.9; 864 x 2560 x 4096 128x128 21 / 96x96 17.0; 1024 x 2560 x 9728 128x128 48.3 / 96x128
+// 41.3; 32 x 19456 x 2560 64x128 15.9 / 64x96 13.7, at 64 rows 19.5 / 15.3; 128 x 19456 x 2560
+// 128x128 21.4 / 128x96 18.7; 200 x 6144 x 2560 128x64 16 / 64x96 11.1.  Neighbours in the order
+// differ by little (700 x 2560 x 9728: 128x64 30.2, 96x96 31.1, 128x96 36.0, 96x128 36.0).
+constexpr PrefillChoice kSingleWave[] = {{64, 64},  {96, 64},  {64, 96},  {128, 64}, {96, 96},
+                                         {64, 128}, {96, 128}, {128, 96}, {128, 128}};
+
 PrefillChoice prefill_tile(int64_t M, int64_t N, bool rows256_ok) {
   const int64_t cus = device_cus();
-  PrefillChoice c = choose_prefill(M, N, cus, rows256_ok);
-  if (c.rows == 128 && c.bn <= 128 && cdiv(M, 96) * cdiv(N, c.bn) <= cus) c.rows = 96;
+  const PrefillChoice c = choose_prefill(M, N, cus, rows256_ok);
+  if (c.rows > 128 || cdiv(M, c.rows) * cdiv(N, c.bn) > cus) return c;
+  for (const PrefillChoice& t : kSingleWave)
+    if (cdiv(M, t.rows) * cdiv(N, t.bn) <= cus) return t;
   return c;
 }
 }  // namespace

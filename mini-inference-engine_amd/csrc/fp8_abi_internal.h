@@ -77,7 +77,8 @@ int launch_norm_gate_up_silu(const uint16_t* x, int64_t sxm, const uint16_t* res
 // activation codes are zero up to a whole group past K) K may be any multiple of 16.
 bool tile_dma_supported(const uint8_t* q, int64_t ldq, int64_t as_sm, int64_t as_sk, const uint8_t* w,
                         int64_t ldw, int64_t M, int64_t K, bool q_padded);
-// bn: tile width, 64, 128 or 160; rows: tile rows, 128, or 96 or 64 (widths 64 and 128).
+// bn: tile width, 64, 96, 128 or 160; rows: tile rows, 128, or 96 or 64 (widths to 128).  96 rows or
+// columns only where the tiles fit one per CU.
 int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_sk, const uint8_t* w,
                     int64_t ldw, const float* ws, int64_t ws_sn, int64_t ws_sk, void* out, int out_dtype,
                     int64_t ldo, int64_t M, int64_t N, int64_t K, int bn, int rows, hipStream_t stream,

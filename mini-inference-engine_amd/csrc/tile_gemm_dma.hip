@@ -3,8 +3,8 @@
 // Same arithmetic and lane layout as tile_gemm_kernel (block_gemm.hip): one
 // v_mfma_f32_16x16x128_f8f6f4 per 128-wide K group and 16x16 output tile, folded into the
 // fp32 accumulator as acc = fma(partial, a_s * w_s, acc); 128 x BN output tile per
-// 256-thread workgroup (BN = 64, 128 or 160), 2x2 waves of 64 x BN/2, and the same with 96 or
-// 64 rows (BN = 64 or 128).  BN = 160 gives the
+// 256-thread workgroup (BN = 64, 96, 128 or 160), 2x2 waves of 64 x BN/2, and the same with 96
+// or 64 rows (BN to 128).  BN = 160 gives the
 // Qwen3-4B o_proj and down projections at M = 2048 exactly 256 tiles (16 x 16) instead
 // of 320; a wave's columns may then straddle two 128-column weight-scale blocks, so each
 // 16-column MFMA tile uses its own block's scale.
@@ -60,11 +60,11 @@ constexpr int kStagesMany = 2;  // otherwise (two workgroups per CU)
 constexpr int kTileRows = 128;                          // activation rows per tile
 constexpr int kMaxBN = 160;                             // widest W tile (columns of the output tile)
 
-// Tile geometry for width BN (64, 128 or 160) and J 16-row activation fragments per wave
-// (tile rows 32 J: 128 for J = 4, 64 for J = 2): stage layout [W tile | X tile | scales].
+// Tile geometry for width BN (64, 96, 128 or 160) and J 16-row activation fragments per wave
+// (tile rows 32 J: 128 for J = 4, 96 for J = 3, 64 for J = 2): stage layout [W tile | X tile | scales].
 template <int BN, int J = 4>
 struct DmaGeo {
-  static_assert(BN == 64 || BN == 128 || BN == 160, "tile width");
+  static_assert(BN == 64 || BN == 96 || BN == 128 || BN == 160, "tile width");
   static_assert(J == 4 || (J == 3 && BN != 160) || J == 2, "tile rows");
   static constexpr int kNI = BN / 32;                  // 16-column MFMA tiles per wave (2 x 2 waves)
   static constexpr int kRows = 32 * J;                 // activation rows of the tile
@@ -388,9 +388,9 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
   tile_of_dma(blockIdx.x, tiles_m, tiles_n, &tm, &tn);
   using G = DmaGeo<BN, J>;
   constexpr int NI = G::kNI;
-  // A wave's columns lie in one 128-column weight-scale block unless BN = 160, or the up half
+  // A wave's columns lie in one 128-column weight-scale block unless BN = 160 or 96, or the up half
   // starts inside one.
-  constexpr bool kTwo = BN == 160 || SILU;
+  constexpr bool kTwo = BN == 160 || BN == 96 || SILU;
   const int64_t m0 = tm * G::kRows;
   // SILU: the tile's first BN / 2 weight rows are gate rows n0 .., the rest up rows N / 2 + n0 ...
   const int64_t half = N / 2;
@@ -512,7 +512,6 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
     }
     __syncthreads();
     constexpr int C = (SILU ? BN / 2 : BN) / 8;  // 16-byte pieces per row
-    static_assert((G::kRows * BN / 8) % kDmaThreads == 0, "whole passes");
     const int64_t n_end = SILU ? half : N;
 #pragma unroll
     for (int idx = tid; idx < G::kRows * C; idx += kDmaThreads) {
@@ -566,7 +565,7 @@ bool tile_dma_supported(const uint8_t* q, int64_t ldq, int64_t as_sm, int64_t as
 int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_sk, const uint8_t* w,
                     int64_t ldw, const float* ws, int64_t ws_sn, int64_t ws_sk, void* out, int out_dtype,
                     int64_t ldo, int64_t M, int64_t N, int64_t K, int bn, int rows, hipStream_t stream, bool silu) {
-  if (bn != 64 && bn != 128 && bn != 160) return MI355X_FP8_ERR_INVALID;
+  if (bn != 64 && bn != 96 && bn != 128 && bn != 160) return MI355X_FP8_ERR_INVALID;
   if (rows != 128 && ((rows != 64 && rows != 96) || bn == 160)) return MI355X_FP8_ERR_INVALID;
   const int64_t tiles_m = (M + rows - 1) / rows;
   const int64_t tiles_n = (N + bn - 1) / bn;
@@ -581,6 +580,7 @@ int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_s
   // flight; six, where they fit, measured the same (28.0 and 28.3 us for N = 2560, K = 9728 at
   // 536 rows).  64x64 tiles have room for two workgroups of four stages.
   const bool few = tiles_m * tiles_n <= device_cus();
+  if (!few && (rows == 96 || bn == 96)) return MI355X_FP8_ERR_INVALID;
 #define MI355X_DMA_ARGS q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, o, ldo, M, N, (K + kGroup - 1) / kGroup, tiles_m, tiles_n, vec_out, tail
 #define MI355X_DMA_LAUNCH_T(ST, BN, T, J, KT, SI) \
   tile_gemm_dma_kernel<ST, BN, T, J, KT, SI><<<grid, kDmaThreads, 0, stream>>>(MI355X_DMA_ARGS)
@@ -596,13 +596,15 @@ int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_s
   } while (0)
   if (rows == 64) {
     if (bn == 64) MI355X_DMA_LAUNCH(kStagesFew, 64, 2);
+    else if (bn == 96) MI355X_DMA_LAUNCH(kStagesFew, 96, 2);
     else MI355X_DMA_ROWS(128, 2);
   } else if (rows == 96) {
-    if (!few) return MI355X_FP8_ERR_INVALID;
     if (bn == 64) MI355X_DMA_LAUNCH(kStagesFew, 64, 3);
+    else if (bn == 96) MI355X_DMA_LAUNCH(kStagesFew, 96, 3);
     else MI355X_DMA_LAUNCH(kStagesFew, 128, 3);
   } else {
     if (bn == 160) MI355X_DMA_ROWS(160, 4);
+    else if (bn == 96) MI355X_DMA_LAUNCH(kStagesFew, 96, 4);
     else if (bn == 64) MI355X_DMA_ROWS(64, 4);
     else MI355X_DMA_ROWS(128, 4);
   }

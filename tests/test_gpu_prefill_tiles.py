@@ -26,9 +26,12 @@ def _reference(x, w, ws, out_dtype):
     # 96-row tiles (128-row picks whose 96-row form fits one per CU), rows at their edges.
     (512, 2560, 512), (536, 2560, 384), (385, 2500, 640), (577, 2560, 128), (97, 6144, 1024), (1024, 2560, 256),
     (1056, 2560, 896),
+    # 96-wide tiles at every tile height, whose column halves straddle weight-scale blocks.
+    (200, 6144, 384), (32, 19456, 256), (63, 19400, 128), (128, 19456, 640), (100, 11008, 512), (864, 2560, 256),
+    (865, 2570, 384),
     # K ending inside a group (16 to 112 columns of it), one group and several, every tile height.
     (333, 2880, 2880), (96, 320, 16), (65, 192, 112), (128, 129, 144), (300, 2560, 400), (700, 3000, 1200),
-    (2048, 2560, 656), (1500, 6144, 336), (40, 12800, 272),
+    (2048, 2560, 656), (1500, 6144, 336), (40, 12800, 272), (200, 6144, 400), (864, 2500, 176), (128, 19456, 208),
 ])
 def test_linear_equals_register_kernel(m, n, k, dtype):
     shape = ModelShape("tiles", n, k)
