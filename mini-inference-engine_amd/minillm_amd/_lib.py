@@ -8,11 +8,12 @@ streams and device pointers are valid arguments.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 
 import torch  # noqa: F401  (must load the HIP runtime before the library)
 
-from .build import LIB_PATH
+from .build import LIB_PATH, TORCH_PATH
 
 _i64 = ctypes.c_int64
 _int = ctypes.c_int
@@ -89,6 +90,27 @@ def load() -> ctypes.CDLL:
             raise RuntimeError("libmi355x_fp8.so ABI version mismatch; rebuild it")
         _lib = lib
     return _lib
+
+
+_native = None
+
+
+def load_native():
+    """The native side of the Python wrapper's common case (``lib/_torch_linear.so``), loaded
+    once.  It links the HIP library, so that is loaded (and checked) first."""
+
+    global _native
+    if _native is None:
+        load()
+        if not os.path.exists(TORCH_PATH):
+            raise RuntimeError(
+                f"{TORCH_PATH} is missing: build it with `python -m minillm_amd.build` "
+                "(there is no fallback implementation)")
+        spec = importlib.util.spec_from_file_location("_torch_linear", TORCH_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _native = module
+    return _native
 
 
 def check(status: int) -> None:

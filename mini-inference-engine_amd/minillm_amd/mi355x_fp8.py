@@ -363,6 +363,15 @@ def mi355x_fp8_linear(
     ``allow_deepgemm`` is accepted and ignored, as in the reference's fast path.
     """
 
+    if (gemm_config is None and activation_scale is None and path in ("auto", "fused", "split")
+            and type(block_size) in (list, tuple) and tuple(block_size) == SUPPORTED_BLOCK_SIZE
+            and isinstance(input, torch.Tensor) and isinstance(weight, torch.Tensor)
+            and isinstance(weight_scale_inv, torch.Tensor) and input.is_cuda):
+        # The common case in one native call; None for anything it leaves to the code below.
+        result = (_lib._native or _lib.load_native()).linear(input, weight, weight_scale_inv, output_dtype,
+                                                             _workspace._buffers)
+        if result is not None:
+            return result if bias is None else result + bias
     select_fp8_path(0, path)  # reject typos first
     if gemm_config is not None and (path != "split" or gemm_config not in GEMM_CONFIGS):
         raise ValueError("gemm_config must be a listed GEMM config with path='split'")
