@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kQuantThreads) void act_quant_wide_kernel(
 #pragma unroll
   for (int i = 0; i < E; ++i) amax = fmaxf(amax, fabsf(t[i]));
   amax = group_max<L>(amax);
-  const float scale = amax / 448.0f;
+  const float scale = scale_of(amax);
   const float den = scale > 1e-12f ? scale : 1e-12f;
   uint32_t packed[E / 4];
   quant_codes<E>(t, den, packed);

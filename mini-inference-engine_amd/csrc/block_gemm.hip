@@ -445,7 +445,7 @@ __global__ __launch_bounds__(kStreamWaves * 64) void stream_gemm_kernel(
       // The four lanes of a token (g = 0..3, lanes r + 16 g) hold the whole group.
       amax = row_max(amax);
     }
-    const float scale = amax / 448.0f;
+    const float scale = scale_of(amax);
     const float den = scale > 1e-12f ? scale : 1e-12f;
     uint32_t packed[kN / 4];
     quant_codes<kN>(t, den, packed);

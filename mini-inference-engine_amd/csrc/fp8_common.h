@@ -150,6 +150,22 @@ __device__ __forceinline__ float div_by_scale(float t, float den, float r) {
   return __builtin_copysignf(__builtin_fmaf(rem, r, q0), t);
 }
 
+// amax / 448, correctly rounded, by div_by_scale's remainder correction with a constant reciprocal
+// (an infinity stays one), and 1 / den for a finite den >= 1e-12, by one Newton step on the
+// hardware reciprocal: 5 and 3 issue slots instead of the 11 and 10 of the divisions.  Both were
+// compared with IEEE division over every amax that a group of bf16 or fp16 values can have (and the
+// den it gives): equal bits.
+__device__ __forceinline__ float scale_of(float amax) {
+  constexpr float r = 1.0f / 448.0f;
+  const float q0 = amax * r;
+  const float q = __builtin_fmaf(__builtin_fmaf(-448.0f, q0, amax), r, q0);
+  return amax < __builtin_inff() ? q : amax;
+}
+__device__ __forceinline__ float recip_den(float den) {
+  const float r = __builtin_amdgcn_rcpf(den);
+  return __builtin_fmaf(__builtin_fmaf(-den, r, 1.0f), r, r);
+}
+
 // Codes of 4 consecutive elements t[0..3] scaled by den (r = 1 / den when den is finite).
 template <bool FAST>
 __device__ __forceinline__ uint32_t quant4(const float* t, float den, float r) {
@@ -164,7 +180,7 @@ __device__ __forceinline__ uint32_t quant4(const float* t, float den, float r) {
 template <int N>
 __device__ __forceinline__ void quant_codes(const float* t, float den, uint32_t* packed) {
   if (__builtin_isfinite(den)) {
-    const float r = 1.0f / den;
+    const float r = recip_den(den);
 #pragma unroll
     for (int i = 0; i < N / 4; ++i) packed[i] = quant4<true>(t + 4 * i, den, r);
   } else {
@@ -185,19 +201,24 @@ __device__ __forceinline__ float row_partner32(float x) {
   return __uint_as_float(((__lane_id() >> 5) & 1) ? v[0] : v[1]);
 }
 
-// The halving tree s[t] += s[t + h], h = 32, 16, ..., 1, over the 64 lanes, with lane-to-lane
-// VALU moves instead of LDS shuffles: v_permlane32_swap and v_permlane16_swap bring lanes
-// t + 32 and t + 16 to lanes t, DPP row_shl:h brings t + h within each 16-lane row.  Lane t < h
-// adds lane t + h's value at every step, so lane 0 ends with the tree's sum, which goes to
-// every lane.
-__device__ __forceinline__ float tree_sum64(float s) {
-  s = s + __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(s), __float_as_uint(s), false, false)[1]);
+// tree_sum64's steps h = 16, 8, ..., 1, over lanes 0 .. 31.
+__device__ __forceinline__ float tree_sum32(float s) {
   s = s + __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(s), __float_as_uint(s), false, false)[1]);
   s = s + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x108, 0xf, 0xf, true));  // row_shl:8
   s = s + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x104, 0xf, 0xf, true));  // row_shl:4
   s = s + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x102, 0xf, 0xf, true));  // row_shl:2
   s = s + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x101, 0xf, 0xf, true));  // row_shl:1
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), 0));
+}
+
+// The halving tree s[t] += s[t + h], h = 32, 16, ..., 1, over the 64 lanes, with lane-to-lane
+// VALU moves instead of LDS shuffles: v_permlane32_swap and v_permlane16_swap bring lanes
+// t + 32 and t + 16 to lanes t, DPP row_shl:h brings t + h within each 16-lane row.  Lane t < h
+// adds lane t + h's value at every step, so lane 0 ends with the tree's sum, which goes to
+// every lane.
+__device__ __forceinline__ float tree_sum64(float s) {
+  return tree_sum32(
+      s + __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(s), __float_as_uint(s), false, false)[1]));
 }
 
 // The maximum over each aligned group of L consecutive lanes (L a power of two), in every lane
@@ -234,7 +255,7 @@ __device__ __forceinline__ float quant_group16(const float (&t)[8], uint32_t (&p
 #pragma unroll
   for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(t[i]));
   amax = group_max<16>(amax);
-  const float scale = amax / 448.0f;
+  const float scale = scale_of(amax);
   const float den = scale > 1e-12f ? scale : 1e-12f;
   quant_codes<8>(t, den, packed);
   return scale;

@@ -24,12 +24,17 @@
 // ((a0 + a1) + a2) + a3; then threads fold pairwise, s_t += s_{t+h} for h = bw/2, ..., 1.
 //
 // Layout: a workgroup of 4 waves holds 4 / wpr rows, each row spread over wpr waves (4 for
-// up to 256 rows, 2 up to 512, else 1; the reduction order does not depend on wpr).  The
+// up to 512 rows, else 2; the reduction order does not depend on wpr).  The
 // norm weight and the rows are read once into LDS (rows up to 16128 wide).  Virtual thread
-// t of the reduction lives in lane t % 64 of the row's wave (t / 64) % wpr, so folds with
+// t of the reduction lives in lane t % 64 of the row's wave (t / 64) % wpr (reductions of 32
+// threads, 16 rows and more: in every wave, two lanes each), so folds with
 // h >= 64 wpr stay inside a lane, folds between 64 and 64 wpr go through LDS, and the rest
 // are shuffles.  The second pass normalizes and quantizes one 128-wide group per 16-lane
 // slice, 8 elements per lane.
+// A latency chain (load, reduce, normalize, store) on few waves per SIMD, not bandwidth, bounds it:
+// with every wave of a row forming the whole sum from reads issued ahead, no redundant loads and
+// the quantizer's short divisions, 32 rows x 2560 with the residual went from 6.3 to 4.8 us, 2048
+// rows from 13.1 to 11.5 (3.2 TB/s).
 // HBM traffic per row: 2K bytes in (4K with the residual), K + 4K/128 out (+2K for the
 // residual sum).
 #include "fp8_abi_internal.h"
@@ -39,7 +44,6 @@ namespace mi355x {
 namespace {
 
 constexpr int kRnqWavesPerBlock = 4;
-constexpr int kRnqBatch = 8;                // 16-byte loads in flight per lane
 constexpr int64_t kRnqLdsBytes = 64 * 1024;  // weight, row buffers and fold buffer of one workgroup
 
 extern __shared__ uint16_t rnq_lds[];  // [K] norm weight, then [rows per block][K] rows after the residual add
@@ -50,7 +54,9 @@ __device__ __forceinline__ float bf16_val(uint16_t b) { return __uint_as_float(s
 // LDS once, 16-byte loads when aligned; both passes then read LDS: pass 1 in the
 // reduction's order, pass 2 one 128-wide group per 16-lane slice.  One workgroup barrier
 // separates the loads from both passes.
-template <bool RESIDUAL>
+// kRnqBatch: 16-byte loads in flight per lane (the fewest of 2, 5 and 8 that hold a row, so that
+// no lane loads the clamped last piece of the row again and again).
+template <bool RESIDUAL, int kRnqBatch>
 __global__ __launch_bounds__(64 * kRnqWavesPerBlock) void rmsnorm_quant_kernel(
     const uint16_t* __restrict__ x, int64_t sxm, const uint16_t* __restrict__ res, int64_t ldr,
     uint16_t* __restrict__ res_out, int64_t ldro, const uint16_t* __restrict__ weight, float eps, float inv_k,
@@ -134,57 +140,85 @@ __global__ __launch_bounds__(64 * kRnqWavesPerBlock) void rmsnorm_quant_kernel(
   // Waves past the last row run it on whatever their LDS holds and discard the result: every
   // wave has to reach the barrier below.
   const int64_t nvec = K / 4;
-  const int span = 64 * wpr;  // virtual threads per slot
-  float part[8];              // bw <= 512: at most 8 slots per lane
+  float ssum;
+  if (bw == 32) {
+    // 16 rows and more of a wide row: 32 virtual threads.  Every wave of the row forms the whole
+    // sum, so nothing is exchanged between waves; lane l holds accumulators 2 h and 2 h + 1 (h =
+    // l / 32) of thread l % 32, whose vectors are read kAhead at a time ahead of the chain.
+    constexpr int kAhead = 10;
+    const uint16_t* mine = row + 2 * (lane >> 5);
+    float a0 = 0.0f, a1 = 0.0f;
+    for (int64_t v0 = lane & 31; v0 < nvec; v0 += 32 * kAhead) {
+      uint32_t e[kAhead];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    part[j] = 0.0f;
-    const int t = rl + span * j;
-    if (t >= bw) continue;
-    float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int64_t v = t; v < nvec; v += bw) {
-      const uint2 pair = *reinterpret_cast<const uint2*>(row + 4 * v);
-      const float e[4] = {bf16_val(pair.x & 0xffffu), bf16_val(pair.x >> 16), bf16_val(pair.y & 0xffffu),
-                          bf16_val(pair.y >> 16)};
+      for (int i = 0; i < kAhead; ++i)
+        e[i] = v0 + 32 * i < nvec ? *reinterpret_cast<const uint32_t*>(mine + 4 * (v0 + 32 * i)) : 0u;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = __fadd_rn(a[i], __fmul_rn(e[i], e[i]));
+      for (int i = 0; i < kAhead; ++i) {  // a vector past the row adds squares of +0: no change
+        const float lo = bf16_val(e[i] & 0xffffu), hi = bf16_val(e[i] >> 16);
+        a0 = __fadd_rn(a0, __fmul_rn(lo, lo));
+        a1 = __fadd_rn(a1, __fmul_rn(hi, hi));
+      }
     }
-    part[j] = __fadd_rn(__fadd_rn(__fadd_rn(a[0], a[1]), a[2]), a[3]);
-  }
-  // Folds with h >= 64 wpr: slots j and j + h / (64 wpr) of the same lane.
-  for (int h = bw / 2; h >= span; h >>= 1) {
-    const int hj = h / span;
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (j < hj) part[j] = __fadd_rn(part[j], part[j + hj]);
-  }
-  // Folds with 64 <= h < 64 wpr: the same lane of waves sub and sub + h / 64, through LDS.
-  float ssum = part[0];
-  if (wpr > 1) {
-    red[rl] = ssum;
-    __syncthreads();
-    const int nsub = bw >= span ? wpr : (bw >= 64 ? bw / 64 : 1);
-    float v[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = i < nsub ? red[i * 64 + lane] : 0.0f;
-    for (int h = nsub / 2; h >= 1; h >>= 1) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        if (i < h) v[i] = __fadd_rn(v[i], v[i + h]);
-    }
-    ssum = v[0];
-  }
-  if (!live) return;  // no barrier follows
-  // Folds with h < 64: lane l adds lane l + h (tree_sum64: lane swaps and DPP; a reduction
-  // narrower than a wave keeps the shuffles).
-  if (bw >= 64) {
-    ssum = tree_sum64(ssum);
+    // ((a0 + a1) + a2) + a3 in lanes 0 .. 31 (a2, a3 from lane + 32), then s[t] += s[t + h].
+    const auto upper = [](float x) {
+      return __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false)[1]);
+    };
+    ssum = tree_sum32(__fadd_rn(__fadd_rn(__fadd_rn(a0, a1), upper(a0)), upper(a1)));
+    if (!live) return;  // no barrier follows
   } else {
-    for (int h = bw / 2; h >= 1; h >>= 1) {
-      const float other = __shfl_down(ssum, h, 64);
-      if (lane < h) ssum = __fadd_rn(ssum, other);
+    const int span = 64 * wpr;  // virtual threads per slot
+    float part[8];              // bw <= 512: at most 8 slots per lane
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      part[j] = 0.0f;
+      const int t = rl + span * j;
+      if (t >= bw) continue;
+      float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      for (int64_t v = t; v < nvec; v += bw) {
+        const uint2 pair = *reinterpret_cast<const uint2*>(row + 4 * v);
+        const float e[4] = {bf16_val(pair.x & 0xffffu), bf16_val(pair.x >> 16), bf16_val(pair.y & 0xffffu),
+                            bf16_val(pair.y >> 16)};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[i] = __fadd_rn(a[i], __fmul_rn(e[i], e[i]));
+      }
+      part[j] = __fadd_rn(__fadd_rn(__fadd_rn(a[0], a[1]), a[2]), a[3]);
     }
-    ssum = __shfl(ssum, 0, 64);
+    // Folds with h >= 64 wpr: slots j and j + h / (64 wpr) of the same lane.
+    for (int h = bw / 2; h >= span; h >>= 1) {
+      const int hj = h / span;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (j < hj) part[j] = __fadd_rn(part[j], part[j + hj]);
+    }
+    // Folds with 64 <= h < 64 wpr: the same lane of waves sub and sub + h / 64, through LDS.
+    ssum = part[0];
+    if (wpr > 1) {
+      red[rl] = ssum;
+      __syncthreads();
+      const int nsub = bw >= span ? wpr : (bw >= 64 ? bw / 64 : 1);
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = i < nsub ? red[i * 64 + lane] : 0.0f;
+      for (int h = nsub / 2; h >= 1; h >>= 1) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          if (i < h) v[i] = __fadd_rn(v[i], v[i + h]);
+      }
+      ssum = v[0];
+    }
+    if (!live) return;  // no barrier follows
+    // Folds with h < 64: lane l adds lane l + h (tree_sum64: lane swaps and DPP; a reduction
+    // narrower than a wave keeps the shuffles).
+    if (bw >= 64) {
+      ssum = tree_sum64(ssum);
+    } else {
+      for (int h = bw / 2; h >= 1; h >>= 1) {
+        const float other = __shfl_down(ssum, h, 64);
+        if (lane < h) ssum = __fadd_rn(ssum, other);
+      }
+      ssum = __shfl(ssum, 0, 64);
+    }
   }
   const float var = __fmul_rn(ssum, inv_k);
   const float inv = static_cast<float>(1.0 / sqrt(static_cast<double>(__fadd_rn(var, eps))));
@@ -271,8 +305,10 @@ int launch_rmsnorm_quant(const uint16_t* x, int64_t sxm, const uint16_t* res, in
   const int64_t row_bytes = 2 * K;
   if (2 * row_bytes + 1024 > kRnqLdsBytes) return MI355X_FP8_ERR_UNSUPPORTED;  // K > 16128
   // Waves per row: few rows spread each over several waves (the reduction order does not
-  // depend on it), so that more of the chip works on them.
-  const int wpr = M <= 256 ? 4 : (M <= 512 ? 2 : 1);
+  // depend on it), so that more of the chip works on them.  Measured with the residual, K = 2560
+  // (us, 1 or 2 / 4 waves): 512 rows 5.9 / 5.6; (1 / 2 / 4 waves) 1024 rows 8.0 / 7.6 / 7.7, 2048
+  // 11.6 / 11.5 / 13.0, 4096 19.4 / 19.1 / 22.8.
+  const int wpr = M <= 512 ? 4 : 2;
   int rows = static_cast<int>((kRnqLdsBytes - 1024) / row_bytes) - 1;  // the weight and the fold buffer
   rows = rows < kRnqWavesPerBlock / wpr ? rows : kRnqWavesPerBlock / wpr;
   const int64_t blocks = (M + rows - 1) / rows;
@@ -285,13 +321,21 @@ int launch_rmsnorm_quant(const uint16_t* x, int64_t sxm, const uint16_t* res, in
   const float inv_k = 1.0f / static_cast<float>(K);
   const dim3 grid(static_cast<unsigned>(blocks));
   const size_t lds = static_cast<size_t>(rows + 1) * row_bytes + static_cast<size_t>(rows) * 64 * wpr * 4;
-  if (res != nullptr)
-    rmsnorm_quant_kernel<true><<<grid, 64 * rows * wpr, lds, stream>>>(x, sxm, res, ldr, res_out, ldro, weight, eps, inv_k,
-                                                                 M, K, bw, rows, wpr, vec, y, ldy, q, ldq, kpad, s, ssm, ssk);
-  else
-    rmsnorm_quant_kernel<false><<<grid, 64 * rows * wpr, lds, stream>>>(x, sxm, res, ldr, res_out, ldro, weight, eps,
-                                                                  inv_k, M, K, bw, rows, wpr, vec, y, ldy, q, ldq, kpad, s,
-                                                                  ssm, ssk);
+  const int64_t pieces = (K / 8 + 64 * wpr - 1) / (64 * wpr);  // 16-byte pieces of a row per lane
+#define MI355X_RNQ(RES, B)                                                                                            \
+  rmsnorm_quant_kernel<RES, B><<<grid, 64 * rows * wpr, lds, stream>>>(x, sxm, res, ldr, res_out, ldro, weight, eps, inv_k, \
+                                                                       M, K, bw, rows, wpr, vec, y, ldy, q, ldq, kpad, s,   \
+                                                                       ssm, ssk)
+#define MI355X_RNQ_BATCH(RES)               \
+  do {                                      \
+    if (pieces <= 2) MI355X_RNQ(RES, 2);    \
+    else if (pieces <= 5) MI355X_RNQ(RES, 5); \
+    else MI355X_RNQ(RES, 8);                \
+  } while (0)
+  if (res != nullptr) MI355X_RNQ_BATCH(true);
+  else MI355X_RNQ_BATCH(false);
+#undef MI355X_RNQ_BATCH
+#undef MI355X_RNQ
   return hipGetLastError() == hipSuccess ? MI355X_FP8_OK : MI355X_FP8_ERR_LAUNCH;
 }
 
