@@ -319,7 +319,8 @@ def _gemm_silu_takes(m: int, k: int, weight: torch.Tensor, scales: torch.Tensor,
     the separate GEMM and SiLU*up, which raise what they raise."""
 
     return bool(
-        m > 16 and k % 128 == 0 and weight.ndim == 2 and scales.ndim == 2 and weight.shape[0] % 32 == 0
+        m > 16 and k and k % 128 == 0 and weight.ndim == 2 and scales.ndim == 2
+        and weight.shape[0] and weight.shape[0] % 32 == 0
         and weight.shape[1] == k and weight.dtype == torch.float8_e4m3fn and scales.dtype == torch.float32
         and weight.stride(1) == 1 and weight.stride(0) >= k and weight.device == scales.device == device
         and tuple(scales.shape) == (-(-weight.shape[0] // 128), k // 128)
@@ -751,8 +752,8 @@ def mlp_forward_mi355x_fp8(x: torch.Tensor, gate_up_weight: torch.Tensor, gate_u
     k = int(x.shape[-1])
     x2 = x.reshape(-1, k)
     h = None
-    if (x.dtype == torch.bfloat16 and _supports_call(x2, gate_up_weight, gate_up_scale, SUPPORTED_BLOCK_SIZE, None)
-            and _gemm_silu_takes(x2.shape[0], k, gate_up_weight, gate_up_scale, x.device)):
+    if (x.dtype == torch.bfloat16 and _gemm_silu_takes(x2.shape[0], k, gate_up_weight, gate_up_scale, x.device)
+            and _supports_call(x2, gate_up_weight, gate_up_scale, SUPPORTED_BLOCK_SIZE, None)):
         q, s = quantize_mi355x_fp8_activation(x2, scale_layout="kgroup")
         h = _gemm_silu(q, s, gate_up_weight, gate_up_scale)
     if h is not None:
