@@ -11,7 +11,7 @@
 //
 // What differs is the feed: global memory goes straight into LDS with
 // global_load_lds_dwordx4 (no register staging, no ds_write), through a ring of STAGES
-// stages (2 when two workgroups share a CU, else 4).  Each stage holds the W tile (BN rows x 128 B), the activation tile
+// stages (2 when two workgroups share a CU, else 4, or 3 at width 160).  Each stage holds the W tile (BN rows x 128 B), the activation tile
 // (128 x 128 B) and the 128 activation scales of its K group.  A 64-lane DMA instruction fills 1 KiB of LDS
 // linearly (lane i -> byte 16 i), i.e. 8 rows of 8 16-byte chunks; the XOR swizzle
 // (physical chunk p of row r holds logical chunk p ^ (r & 7)) is applied by choosing each
@@ -24,10 +24,11 @@
 // K = 9728 at 536 rows a step takes 0.33 us, 0.24 us without the DMA and 0.11 us of MFMA; more
 // stages, no barrier and no fold each change it by less than 4 %.  Measured against the former
 // step, which read the fragments of its first MFMAs during the previous step only (us, weights
-// from HBM): N = 2560 at 536 rows K = 4096 17.1 -> 14.3, K = 9728 32.6 -> 28.0; at 2048 rows
-// (128x160) 59.1 -> 57.9.
+// from HBM): N = 2560 at 536 rows K = 4096 17.1 -> 14.3, K = 9728 32.6 -> 28.0.
 // Two workgroups per CU (two stages, k_step; also 256 registers at most): the two hide each
-// other's waits; a K step reads the fragments of its first MFMAs during the previous step, each
+// other's waits.  The 160-wide single waves (three stages) keep this step too: twenty MFMAs a step
+// hide most of the reads already, and the other step measured 29.5 against 28.5 us (N = 2560, K =
+// 4096 at 2048 rows, weights from HBM; K = 9728 the same).  A K step reads the fragments of its first MFMAs during the previous step, each
 // later weight fragment while the MFMAs of the one before run, and the barrier sits between the
 // two parts.  The K loop is unrolled by STAGES so that every stage index is a compile-time
 // constant.
@@ -56,6 +57,7 @@ namespace {
 
 constexpr int kDmaThreads = 256;
 constexpr int kStagesFew = 4;   // ring depth when the tiles do not exceed the CUs
+constexpr int kStagesFew160 = 3;  // the same for the 160-wide tiles, with the two-part k_step
 constexpr int kStagesMany = 2;  // otherwise (two workgroups per CU)
 constexpr int kTileRows = 128;                          // activation rows per tile
 constexpr int kMaxBN = 160;                             // widest W tile (columns of the output tile)
@@ -445,26 +447,27 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
 #pragma unroll
     for (int j = 0; j < J; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
-  static_assert(STAGES == 2 || STAGES == 4, "stages");
+  static_assert(STAGES >= 2 && STAGES <= 4, "stages");
   issue_stage<BN, 0, J, KTAIL>(ring, src, 0, KB, as_sk, wave);
   issue_stage<BN, 1, J, KTAIL>(ring, src, KB > 1 ? 1 : KB - 1, KB, as_sk, wave);
-  if constexpr (STAGES == 4) {
-    issue_stage<BN, 2, J, KTAIL>(ring, src, KB > 2 ? 2 : KB - 1, KB, as_sk, wave);
-    issue_stage<BN, 3, J, KTAIL>(ring, src, KB > 3 ? 3 : KB - 1, KB, as_sk, wave);
-  }
+  if constexpr (STAGES >= 3) issue_stage<BN, 2, J, KTAIL>(ring, src, KB > 2 ? 2 : KB - 1, KB, as_sk, wave);
+  if constexpr (STAGES >= 4) issue_stage<BN, 3, J, KTAIL>(ring, src, KB > 3 ? 3 : KB - 1, KB, as_sk, wave);
   wait_vm_lgkm0<G::kDmaPerStage * (STAGES - 1)>();
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   int64_t kb = 0;
-  if constexpr (STAGES == 2) {
+  if constexpr (STAGES <= 3) {
     StepHead<BN, J> h;
     read_head<BN, 0, J>(ring, h, src, 0, ws_sk, wm, wn, r, g);
 #define MI355X_KSTEP(S, KBV) k_step<BN, STAGES, S, J, KTAIL, kTwo>(ring, acc, h, src, KBV, KB, as_sk, ws_sk, wave, wm, wn, r, g)
-    for (; kb + 2 <= KB; kb += 2) {
+    for (; kb + STAGES <= KB; kb += STAGES) {
       MI355X_KSTEP(0, kb);
       MI355X_KSTEP(1, kb + 1);
+      if constexpr (STAGES == 3) MI355X_KSTEP(2, kb + 2);
     }
     if (kb < KB) MI355X_KSTEP(0, kb);
+    if constexpr (STAGES == 3)
+      if (kb + 1 < KB) MI355X_KSTEP(1, kb + 1);
 #undef MI355X_KSTEP
   } else {
     StepRegs<BN, J> f0, f1;
@@ -603,7 +606,8 @@ int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_s
     else if (bn == 96) MI355X_DMA_LAUNCH(kStagesFew, 96, 3);
     else MI355X_DMA_LAUNCH(kStagesFew, 128, 3);
   } else {
-    if (bn == 160) MI355X_DMA_ROWS(160, 4);
+    if (bn == 160 && few) MI355X_DMA_LAUNCH(kStagesFew160, 160, 4);
+    else if (bn == 160) MI355X_DMA_LAUNCH(kStagesMany, 160, 4);
     else if (bn == 96) MI355X_DMA_LAUNCH(kStagesFew, 96, 4);
     else if (bn == 64) MI355X_DMA_ROWS(64, 4);
     else MI355X_DMA_ROWS(128, 4);
