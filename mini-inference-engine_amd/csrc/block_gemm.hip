@@ -244,7 +244,7 @@ __device__ __forceinline__ float norm_row_inv(const uint2 (&xv)[kNormMaxVec], in
     for (int j = 0; j < hj; ++j) part[j] = part[j] + part[j + hj];
   const float ss = tree_sum64(part[0]);
   const float var = ss * na.inv_k;
-  return static_cast<float>(1.0 / sqrt(static_cast<double>(var + na.eps)));
+  return rsqrt_rn(var + na.eps);
 }
 
 template <int NT, int AF, bool ALIGNED, bool RAGGED, typename OutT, typename XIn = uint8_t, int QT = 16,

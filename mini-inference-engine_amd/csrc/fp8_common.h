@@ -131,6 +131,18 @@ __device__ __forceinline__ void store8_cols(uint16_t* dst, uint4 v, int64_t n, i
   }
 }
 
+// 1 / sqrt(v) rounded once to fp32, as through double square root and division: the hardware's
+// double reciprocal square root and one third-order Newton step, a chain of 6 operations instead of
+// some 25 in front of everything a norm still has to do.  Compared with (float)(1.0 / sqrt((double)v))
+// over every positive finite fp32 v: equal bits.  Zero, infinity and NaN take that form.
+__device__ __forceinline__ float rsqrt_rn(float v) {
+  const double d = static_cast<double>(v);
+  if (!(v > 0.0f && v < __builtin_inff())) return static_cast<float>(1.0 / sqrt(d));
+  const double y = __builtin_amdgcn_rsq(d);
+  const double e = __builtin_fma(-(d * y), y, 1.0);
+  return static_cast<float>(__builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y));
+}
+
 // Two fp32 -> two OCP e4m3fn codes (round-to-nearest-even), packed into the low 16 bits.
 __device__ __forceinline__ uint32_t cvt_pk_e4m3(float a, float b) {
   return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false)) & 0xffffu;

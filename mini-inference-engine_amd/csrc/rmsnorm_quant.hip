@@ -10,7 +10,7 @@
 //                                      __fadd_rn are plain operators in HIP, so the library is
 //                                      built with -ffp-contract=off; fused, var + eps came out
 //                                      one rounding short and moved y by one ulp near ties)
-//   inv  = 1 / sqrt(var + eps)         here computed in double and rounded once to fp32
+//   inv  = 1 / sqrt(var + eps)         here correctly rounded (rsqrt_rn)
 //   y    = bf16(w * bf16(x * inv))
 //   q, s = the quantizer of y
 // The reference calls libdevice's approximate rsqrt; the correctly rounded value used here
@@ -221,7 +221,7 @@ __global__ __launch_bounds__(64 * kRnqWavesPerBlock) void rmsnorm_quant_kernel(
     }
   }
   const float var = __fmul_rn(ssum, inv_k);
-  const float inv = static_cast<float>(1.0 / sqrt(static_cast<double>(__fadd_rn(var, eps))));
+  const float inv = rsqrt_rn(__fadd_rn(var, eps));
 
   // ---- pass 2: normalize and quantize, one group per 16-lane slice -----------------
   const int lane16 = lane & 15;

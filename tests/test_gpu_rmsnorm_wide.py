@@ -33,3 +33,20 @@ def test_rmsnorm_quant_wide_rows_match_oracle(rows, width, with_residual):
     assert np.array_equal(outs[2].cpu().numpy().view(np.uint32), s_ref.view(np.uint32))
     if with_residual:
         assert np.array_equal(bits16(outs[3].cpu()), summed_ref)
+
+
+def test_rmsnorm_quant_infinite_and_zero_rows():
+    """Rows whose mean square is infinite, NaN or zero (eps 0) keep what 1 / sqrt gives there: 0,
+    NaN and infinity, so NaN where an infinity meets a zero."""
+
+    x = torch.ones((20, 256), dtype=torch.bfloat16)
+    x[3, 7] = float("inf")
+    x[5, 9] = float("nan")
+    x[8] = 0
+    x[11] = 3e38  # the sum of squares overflows
+    w = torch.ones(256, dtype=torch.bfloat16)
+    y = fp8.rmsnorm_quant_mi355x_fp8(x.cuda(), w.cuda(), 0.0, scale_layout="row", return_intermediate=True)[0].cpu().float()
+    ref = x.float() * torch.rsqrt(x.float().square().mean(dim=1, keepdim=True))
+    assert torch.equal(torch.isnan(y), torch.isnan(ref))
+    keep = ~torch.isnan(ref)
+    assert torch.equal(y[keep], ref[keep])
