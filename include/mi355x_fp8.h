@@ -167,19 +167,22 @@ size_t mi355x_fp8_linear_noalloc_scratch_bytes(void);
  * Dispatch introspection, no reference counterpart (for tests and tuning): the prefill
  * kernel the automatic dispatch runs for an M x N output (M above the decode range, LDS-DMA
  * preconditions met) on a device with `cus` CUs, from the table of measured wave times:
- * *rows = tile rows (64 or 128: the LDS-DMA kernel; 192 or 256: the 256-row kernel and its
- * 192-row form), *bn = tile width.  An LDS-DMA tile that fits one per CU is launched as the
- * cheapest of 64, 96 or 128 rows by 64, 96 or 128 columns that still does.  Pure host computation: no device is touched.
+ * *rows = tile rows (64, 96 or 128: the LDS-DMA kernel; 192 or 256: the 256-row kernel and its
+ * 192-row form), *bn = tile width.  It is the tile that is launched: where the table's pick is an
+ * LDS-DMA tile that fits one per CU, the cheapest of 64, 96 or 128 rows by 64, 96 or 128 columns
+ * that still does.  Pure host computation: no device is touched.
  */
 int mi355x_fp8_prefill_choice(int64_t M, int64_t N, int64_t cus, int* rows, int* bn);
 
 /*
  * Dispatch introspection, no reference counterpart (for benchmarks and tests): the kernel
  * family the automatic dispatch of an M x N x K GEMM picks on a device with `cus` CUs, for
- * 16-byte aligned operands with K % 128 == 0.  *kernel = MI355X_FP8_CONFIG_STREAM (the
+ * 16-byte aligned operands (and, where K % 128 != 0, codes padded with zeros to a whole group, as
+ * the linear's are).  *kernel = MI355X_FP8_CONFIG_STREAM (the
  * weight-streaming decode kernel: *rows = weight rows per workgroup, *cols = token rows per
  * slice) or MI355X_FP8_CONFIG_TILE128 (a prefill tile: *rows x *cols as in
- * mi355x_fp8_prefill_choice).  Pure host computation: no device is touched.
+ * mi355x_fp8_prefill_choice; of at most 128 rows where K % 128 != 0, and the register-staged 128 x
+ * 128 kernel where K % 16 != 0).  Pure host computation: no device is touched.
  */
 int mi355x_fp8_dispatch_choice(int64_t M, int64_t N, int64_t K, int64_t cus, int* kernel, int* rows, int* cols);
 

@@ -251,7 +251,7 @@ size_t mi355x_fp8_linear_noalloc_scratch_bytes(void) {
 
 int mi355x_fp8_prefill_choice(int64_t M, int64_t N, int64_t cus, int* rows, int* bn) {
   if (M <= 0 || N <= 0 || cus <= 0 || rows == nullptr || bn == nullptr) return MI355X_FP8_ERR_INVALID;
-  prefill_choice(M, N, cus, rows, bn);
+  prefill_choice(M, N, cus, true, rows, bn);
   return MI355X_FP8_OK;
 }
 
@@ -265,8 +265,10 @@ int mi355x_fp8_dispatch_choice(int64_t M, int64_t N, int64_t K, int64_t cus, int
   if (plan.kernel == MI355X_FP8_CONFIG_STREAM) {
     *rows = plan.rows;
     *cols = 16 * plan.token_tiles;
+  } else if (K % 16 != 0) {  // the register-staged kernel
+    *rows = *cols = 128;
   } else {
-    prefill_choice(M, N, cus, rows, cols);
+    prefill_choice(M, N, cus, K % 128 == 0, rows, cols);
   }
   return MI355X_FP8_OK;
 }

@@ -909,8 +909,7 @@ PrefillChoice choose_prefill(int64_t M, int64_t N, int64_t cus, bool rows256_ok)
 constexpr PrefillChoice kSingleWave[] = {{64, 64},  {96, 64},  {64, 96},  {128, 64}, {96, 96},
                                          {64, 128}, {96, 128}, {128, 96}, {128, 128}};
 
-PrefillChoice prefill_tile(int64_t M, int64_t N, bool rows256_ok) {
-  const int64_t cus = device_cus();
+PrefillChoice prefill_tile(int64_t M, int64_t N, int64_t cus, bool rows256_ok) {
   const PrefillChoice c = choose_prefill(M, N, cus, rows256_ok);
   if (c.rows > 128 || cdiv(M, c.rows) * cdiv(N, c.bn) > cus) return c;
   for (const PrefillChoice& t : kSingleWave)
@@ -919,8 +918,8 @@ PrefillChoice prefill_tile(int64_t M, int64_t N, bool rows256_ok) {
 }
 }  // namespace
 
-void prefill_choice(int64_t M, int64_t N, int64_t cus, int* rows, int* bn) {
-  const PrefillChoice c = choose_prefill(M, N, cus, true);
+void prefill_choice(int64_t M, int64_t N, int64_t cus, bool whole_k, int* rows, int* bn) {
+  const PrefillChoice c = prefill_tile(M, N, cus, whole_k);
   *rows = c.rows;
   *bn = c.bn;
 }
@@ -1032,7 +1031,7 @@ int launch_gate_up_silu(const uint8_t* q, int64_t ldq, const float* as, int64_t 
   if (plan.kernel != MI355X_FP8_CONFIG_TILE128 || N % 32 != 0 || K % kGroup != 0 || out_vec_mode(h, ldh) != 2 ||
       !tile_dma_supported(q, ldq, as_sm, as_sk, w, ldw, M, K, false) || (N / 2 + 256) * ldw > 0xffffffffLL)
     return MI355X_FP8_ERR_UNSUPPORTED;
-  const PrefillChoice c = prefill_tile(M, N, tile256_offsets_ok(ldq, ldw, M, N, K));
+  const PrefillChoice c = prefill_tile(M, N, device_cus(), tile256_offsets_ok(ldq, ldw, M, N, K));
   if (c.rows > 128)
     return launch_tile256(q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, h, kBF16, ldh, M, N, K, c.bn, c.rows, stream, true);
   return launch_tile_dma(q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, h, kBF16, ldh, M, N, K, c.bn, c.rows, stream, true);
@@ -1066,7 +1065,7 @@ int launch_block_gemm(const GemmPlan& plan, const uint8_t* q, int64_t ldq, const
                           tile256_width(M, N, device_cus()), 256, stream);
   }
   if (plan.kernel == MI355X_FP8_CONFIG_TILE128 && dma_ok) {
-    const PrefillChoice c = prefill_tile(M, N, whole && tile256_offsets_ok(ldq, ldw, M, N, K));
+    const PrefillChoice c = prefill_tile(M, N, device_cus(), whole && tile256_offsets_ok(ldq, ldw, M, N, K));
     if (c.rows > 128)
       return launch_tile256(q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, out, out_dtype, ldo, M, N, K, c.bn, c.rows,
                             stream);

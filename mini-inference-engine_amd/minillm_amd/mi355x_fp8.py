@@ -113,8 +113,8 @@ _ARCH_OK: dict[int, bool] = {}  # device index -> is gfx950 (device properties d
 
 def dispatch_name(rows: int, n: int, k: int, cus: int = 256) -> str:
     """The kernel the automatic dispatch runs for an ``rows x n x k`` GEMM on ``cus`` CUs
-    (aligned operands, K % 128 == 0): ``"stream WxT"`` (the weight-streaming decode kernel,
-    W weight rows per workgroup, T token rows per slice) or ``"tile RxC"`` (a prefill tile).
+    (aligned operands): ``"stream WxT"`` (the weight-streaming decode kernel, W weight rows per
+    workgroup, T token rows per slice) or ``"tile RxC"`` (the prefill tile that is launched).
     Host-only: asks the library's planner, touches no device."""
 
     import ctypes

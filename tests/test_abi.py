@@ -104,15 +104,16 @@ def test_read_probe_validates_on_the_host():
     assert lib.mi355x_fp8_read_probe(dummy, 0, dummy, 4096, None) == _lib.OK             # nothing to read
 
 
-# The automatic prefill dispatch's picks on 256 CUs (tile rows, tile width), from the table of
-# measured wave times in block_gemm.hip (choose_prefill): M -> (qkv, o_proj, gate_up, down).
+# The automatic prefill dispatch's tiles on 256 CUs (tile rows, tile width), from the table of
+# measured wave times in block_gemm.hip (choose_prefill), and for a tile of up to 128 rows that fits
+# one per CU the cheapest that still does (prefill_tile): M -> (qkv, o_proj, gate_up, down).
 PREFILL_PICKS = {
-    96: [(64, 64), (64, 64), (128, 128), (64, 64)],
-    160: [(128, 64), (64, 64), (128, 160), (64, 64)],
-    300: [(64, 128), (64, 64), (192, 160), (64, 64)],
-    536: [(128, 128), (128, 64), (192, 256), (128, 64)],
-    864: [(192, 128), (128, 128), (128, 160), (128, 128)],
-    1024: [(192, 160), (128, 128), (256, 160), (128, 128)],
+    96: [(64, 64), (64, 64), (96, 96), (64, 64)],
+    160: [(96, 64), (64, 64), (128, 160), (64, 64)],
+    300: [(96, 96), (64, 64), (192, 160), (64, 64)],
+    536: [(128, 128), (96, 64), (192, 256), (96, 64)],
+    864: [(192, 128), (96, 96), (128, 160), (96, 96)],
+    1024: [(192, 160), (96, 128), (256, 160), (96, 128)],
     2048: [(256, 192), (128, 160), (256, 224), (128, 160)],
     2208: [(256, 224), (192, 128), (256, 256), (192, 128)],
     4096: [(256, 192), (256, 160), (256, 256), (256, 160)],
@@ -121,9 +122,9 @@ PREFILL_PICKS = {
 
 @pytest.mark.parametrize("m", sorted(PREFILL_PICKS))
 def test_prefill_dispatch_picks(m):
-    """The cost model's kernel for each Qwen3-4B projection (host computation only): the
-    M=2048 benchmark shapes, the 192-row tiles past multiples of 256 or 128 (config 5's 536
-    rows for gate_up), the 64-row tiles at small M."""
+    """The tile launched for each Qwen3-4B projection (host computation only): the M=2048
+    benchmark shapes, the 192-row tiles past multiples of 256 or 128 (config 5's 536 rows for
+    gate_up), the smaller tiles at small M."""
 
     lib = _lib.load()
     rows, bn = ctypes.c_int(), ctypes.c_int()
@@ -159,8 +160,9 @@ def test_rmsnorm_linear_rejects_a_residual_sum_over_its_inputs():
 def test_dispatch_choice_names_the_stream_kernel_then_the_prefill_tiles():
     """The automatic dispatch's kernel family (host computation only): the weight-streaming
     kernel at decode sizes (one 16-token slice up to 16 rows; 32-row slices above while the
-    weight rows give few workgroups), then the prefill tile the cost model picks (the same
-    as mi355x_fp8_prefill_choice)."""
+    weight rows give few workgroups), then the prefill tile that is launched (the same as
+    mi355x_fp8_prefill_choice; none of more than 128 rows where K ends inside a group, and the
+    register-staged kernel where K is not whole 16-element pieces)."""
 
     from minillm_amd import mi355x_fp8 as fp8
 
@@ -170,9 +172,13 @@ def test_dispatch_choice_names_the_stream_kernel_then_the_prefill_tiles():
             name = fp8.dispatch_name(m, n, k)
             assert name.startswith("stream ") and name.endswith("x16"), (m, n, name)
     assert [fp8.dispatch_name(32, n, k) for n, k in shapes] == [
-        "stream 24x32", "stream 10x32", "tile 64x128", "stream 16x32"]
+        "stream 24x32", "stream 10x32", "tile 64x96", "stream 16x32"]
     for m in (160, 536, 2048):
         assert [fp8.dispatch_name(m, n, k) for n, k in shapes] == [f"tile {r}x{c}" for r, c in PREFILL_PICKS[m]]
+    assert fp8.dispatch_name(2048, 6144, 2560) == "tile 256x192"
+    assert fp8.dispatch_name(2048, 6144, 2000) == "tile 128x128"
+    assert fp8.dispatch_name(536, 2560, 4000) == "tile 96x64"
+    assert fp8.dispatch_name(2048, 6144, 2001) == "tile 128x128"
     lib = _lib.load()
     a, b, c = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     assert lib.mi355x_fp8_dispatch_choice(0, 2560, 2560, 256, ctypes.byref(a), ctypes.byref(b),
