@@ -123,6 +123,11 @@ int mi355x_fp8_block_gemm_silu(const uint8_t* q, int64_t ldq, const float* as, i
                                const uint8_t* w, int64_t ldw, const float* ws, int64_t ws_sn, int64_t ws_sk, void* h,
                                int64_t ldh, int64_t M, int64_t N, int64_t K, void* stream);
 
+/* 1 when mi355x_fp8_block_gemm_silu takes M rows on this weight (with contiguous codes and
+ * K-group-major scales, as the quantizers write them, and a 16-byte aligned h), else 0, so that a
+ * caller can ask before it quantizes.  Pure host computation: w is not read. */
+int mi355x_fp8_block_gemm_silu_fits(const uint8_t* w, int64_t ldw, int64_t M, int64_t N, int64_t K);
+
 /* Workspace bytes that mi355x_fp8_linear needs: the quantized activations, their scales
  * and the GEMM's workspace.  Same rules as the GEMM workspace. */
 size_t mi355x_fp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int config);

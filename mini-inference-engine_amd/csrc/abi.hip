@@ -203,6 +203,10 @@ int mi355x_fp8_block_gemm_silu(const uint8_t* q, int64_t ldq, const float* as, i
                              K, static_cast<hipStream_t>(stream));
 }
 
+int mi355x_fp8_block_gemm_silu_fits(const uint8_t* w, int64_t ldw, int64_t M, int64_t N, int64_t K) {
+  return M > 0 && N > 0 && K > 0 && ldw >= K && w != nullptr && gate_up_silu_fits(w, ldw, M, N, K);
+}
+
 size_t mi355x_fp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int config) {
   LinearLayout L;
   if (M < 0 || N < 0 || K <= 0 || linear_layout(M, N, K, config, &L) != MI355X_FP8_OK) return 0;

@@ -1019,17 +1019,22 @@ static int launch_typed(const GemmPlan& plan, const uint8_t* q, int64_t ldq, con
   return hipGetLastError() == hipSuccess ? MI355X_FP8_OK : MI355X_FP8_ERR_LAUNCH;
 }
 
+// The prefill tiles only (the stream kernel has no paired form), whole K groups, and halves that
+// start on a 16-column MFMA tile; codes as the quantizers write them meet the DMA's preconditions.
+bool gate_up_silu_fits(const uint8_t* w, int64_t ldw, int64_t M, int64_t N, int64_t K) {
+  GemmPlan plan;
+  return plan_gemm(M, N, K, MI355X_FP8_CONFIG_AUTO, &plan) == MI355X_FP8_OK &&
+         plan.kernel == MI355X_FP8_CONFIG_TILE128 && N % 32 == 0 && K % kGroup == 0 &&
+         tile_dma_supported(nullptr, K, 1, M, w, ldw, M, K, false) && (N / 2 + 256) * ldw <= 0xffffffffLL;
+}
+
 // The prefill kernels on a merged gate/up weight with SiLU(gate) * up applied in the epilogue.
 int launch_gate_up_silu(const uint8_t* q, int64_t ldq, const float* as, int64_t as_sm, int64_t as_sk,
                         const uint8_t* w, int64_t ldw, const float* ws, int64_t ws_sn, int64_t ws_sk, uint16_t* h,
                         int64_t ldh, int64_t M, int64_t N, int64_t K, hipStream_t stream) {
-  GemmPlan plan;
-  const int st = plan_gemm(M, N, K, MI355X_FP8_CONFIG_AUTO, &plan);
-  if (st != MI355X_FP8_OK) return st;
-  // The prefill tiles only (the stream kernel has no paired form), h rows of 16-byte pieces, and
-  // halves that start on a 16-column MFMA tile.
-  if (plan.kernel != MI355X_FP8_CONFIG_TILE128 || N % 32 != 0 || K % kGroup != 0 || out_vec_mode(h, ldh) != 2 ||
-      !tile_dma_supported(q, ldq, as_sm, as_sk, w, ldw, M, K, false) || (N / 2 + 256) * ldw > 0xffffffffLL)
+  // h in rows of 16-byte pieces.
+  if (!gate_up_silu_fits(w, ldw, M, N, K) || out_vec_mode(h, ldh) != 2 ||
+      !tile_dma_supported(q, ldq, as_sm, as_sk, w, ldw, M, K, false))
     return MI355X_FP8_ERR_UNSUPPORTED;
   const PrefillChoice c = prefill_tile(M, N, device_cus(), tile256_offsets_ok(ldq, ldw, M, N, K));
   if (c.rows > 128)

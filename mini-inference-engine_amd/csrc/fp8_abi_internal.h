@@ -50,6 +50,9 @@ int launch_block_gemm(const GemmPlan& plan, const uint8_t* q, int64_t ldq, const
 int launch_gate_up_silu(const uint8_t* q, int64_t ldq, const float* as, int64_t as_sm, int64_t as_sk,
                         const uint8_t* w, int64_t ldw, const float* ws, int64_t ws_sn, int64_t ws_sk, uint16_t* h,
                         int64_t ldh, int64_t M, int64_t N, int64_t K, hipStream_t stream);
+// Whether launch_gate_up_silu takes a call on this weight (with codes from the library's quantizers
+// and an aligned h): host computation only.
+bool gate_up_silu_fits(const uint8_t* w, int64_t ldw, int64_t M, int64_t N, int64_t K);
 
 // The whole linear in one stream-kernel launch (quantization inside), for plans of the stream
 // kernel with one token tile; MI355X_FP8_ERR_UNSUPPORTED (nothing launched) when the call

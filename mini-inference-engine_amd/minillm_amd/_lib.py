@@ -49,6 +49,7 @@ EXPORTS = {
                                _i64, _i64, _i64, _ptr, _size, _int, _ptr], _int),
     "mi355x_fp8_block_gemm_silu": ([_ptr, _i64, _ptr, _i64, _i64, _ptr, _i64, _ptr, _i64, _i64, _ptr, _i64, _i64, _i64,
                                     _i64, _ptr], _int),
+    "mi355x_fp8_block_gemm_silu_fits": ([_ptr, _i64, _i64, _i64, _i64], _int),
     "mi355x_fp8_silu_mul_quant": ([_ptr, _ptr, _int, _i64, _i64, _i64, _ptr, _i64, _ptr, _i64, _i64, _ptr, _i64, _i64,
                                    _ptr], _int),
     "mi355x_fp8_rmsnorm_quant": ([_ptr, _int, _i64, _i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, ctypes.c_float, _ptr,

@@ -314,16 +314,17 @@ def launch_block_gemm(activation: torch.Tensor, weight: torch.Tensor, output: to
 
 
 def _gemm_silu_takes(m: int, k: int, weight: torch.Tensor, scales: torch.Tensor, device: torch.device) -> bool:
-    """Whether a call may go to ``_gemm_silu``: the facts the C-ABI cannot see (as
-    ``_check_gemm_operands`` raises for), more than 16 rows and whole K groups.  Other calls take
-    the separate GEMM and SiLU*up, which raise what they raise."""
+    """Whether a call goes to ``_gemm_silu``, asked before anything is quantized: the facts the
+    C-ABI cannot see (as ``_check_gemm_operands`` raises for), then the library's own rule on the
+    sizes and the alignment.  Other calls take the separate GEMM and SiLU*up, which raise what
+    they raise."""
 
     return bool(
-        m > 16 and k and k % 128 == 0 and weight.ndim == 2 and scales.ndim == 2
-        and weight.shape[0] and weight.shape[0] % 32 == 0
+        m > 16 and weight.ndim == 2 and scales.ndim == 2
         and weight.shape[1] == k and weight.dtype == torch.float8_e4m3fn and scales.dtype == torch.float32
-        and weight.stride(1) == 1 and weight.stride(0) >= k and weight.device == scales.device == device
-        and tuple(scales.shape) == (-(-weight.shape[0] // 128), k // 128)
+        and weight.stride(1) == 1 and weight.device == scales.device == device
+        and tuple(scales.shape) == (-(-weight.shape[0] // 128), -(-k // 128))
+        and _lib.load().mi355x_fp8_block_gemm_silu_fits(weight.data_ptr(), weight.stride(0), m, weight.shape[0], k)
     )
 
 
@@ -721,12 +722,9 @@ def rmsnorm_gate_up_silu_mi355x_fp8(x: torch.Tensor, norm_weight: torch.Tensor, 
         outs = rmsnorm_quant_mi355x_fp8(x, norm_weight, eps, residual)
         q, s = outs[0].reshape(-1, k), outs[1]
         h = _gemm_silu(q, s, gate_up_weight, gate_up_scale)
-        if h is None:
-            gu2 = torch.empty((q.shape[0], n), device=x.device, dtype=torch.bfloat16)
-            launch_block_gemm(q, gate_up_weight, gu2, s, gate_up_scale)
-            h = silu_mul_quant_mi355x_fp8(gu2[:, :inter], gu2[:, inter:], return_intermediate=True)[0]
-        h = h.reshape(*x.shape[:-1], inter)
-        return (h, outs[2]) if residual is not None else h
+        if h is not None:
+            h = h.reshape(*x.shape[:-1], inter)
+            return (h, outs[2]) if residual is not None else h
 
     outs = rmsnorm_linear_mi355x_fp8(x, norm_weight, eps, gate_up_weight, gate_up_scale, residual)
     gu = outs[0] if residual is not None else outs
@@ -752,8 +750,8 @@ def mlp_forward_mi355x_fp8(x: torch.Tensor, gate_up_weight: torch.Tensor, gate_u
     k = int(x.shape[-1])
     x2 = x.reshape(-1, k)
     h = None
-    if (x.dtype == torch.bfloat16 and _gemm_silu_takes(x2.shape[0], k, gate_up_weight, gate_up_scale, x.device)
-            and _supports_call(x2, gate_up_weight, gate_up_scale, SUPPORTED_BLOCK_SIZE, None)):
+    if (x.dtype == torch.bfloat16 and x.is_cuda and mi355x_available(x.device)
+            and _gemm_silu_takes(x2.shape[0], k, gate_up_weight, gate_up_scale, x.device)):
         q, s = quantize_mi355x_fp8_activation(x2, scale_layout="kgroup")
         h = _gemm_silu(q, s, gate_up_weight, gate_up_scale)
     if h is not None:

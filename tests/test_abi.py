@@ -136,6 +136,21 @@ def test_prefill_dispatch_picks(m):
     assert lib.mi355x_fp8_prefill_choice(0, 2560, 256, ctypes.byref(rows), ctypes.byref(bn)) == _lib.ERR_INVALID
 
 
+def test_gemm_silu_fit_follows_the_planner_and_the_alignment():
+    """Which merged gate/up calls the SiLU epilogue takes (host computation only): none where the
+    planner streams, K or the halves end inside a group or MFMA tile, or the weight is unaligned."""
+
+    fits = _lib.load().mi355x_fp8_block_gemm_silu_fits
+    w = 0x10000000
+    assert fits(w, 2560, 24, 19456, 2560) == 1 and fits(w, 2560, 2048, 19456, 2560) == 1
+    assert fits(w, 2560, 24, 6144, 2560) == 0 and fits(w, 2560, 33, 6144, 2560) == 1  # streamed up to 32 rows
+    assert fits(w, 2560, 64, 4096, 2560) == 0 and fits(w, 2560, 65, 4096, 2560) == 1  # and up to 64
+    assert fits(w, 2560, 16, 19456, 2560) == 0 and fits(w, 2560, 0, 19456, 2560) == 0
+    assert fits(w, 2576, 200, 6144, 2576) == 0 and fits(w, 2560, 200, 6160, 2560) == 0
+    assert fits(w + 8, 2560, 200, 6144, 2560) == 0 and fits(w, 2568, 200, 6144, 2560) == 0
+    assert fits(None, 2560, 200, 6144, 2560) == 0 and fits(w, 2432, 200, 6144, 2560) == 0
+
+
 def test_rmsnorm_linear_rejects_a_residual_sum_over_its_inputs():
     """The one-launch norm-linear refuses residual_out overlapping x or residual (every
     workgroup reads them while one writes the sum) before touching the device; a disjoint

@@ -106,6 +106,28 @@ def test_silu_epilogue_refuses_what_it_cannot_take():
     assert fp8._gemm_silu(q, s, w, ws) is None
 
 
+@pytest.mark.parametrize("m,inter,offset", [(24, 3072, 0), (48, 2048, 0), (200, 512, 8), (200, 512, 0)])
+def test_mlp_quantizes_its_input_once(monkeypatch, m, inter, offset):
+    """Where the epilogue does not take the gate/up GEMM (streamed sizes, a weight that is not
+    16-byte aligned) the linear quantizes the input, and nothing else does."""
+
+    k = 256
+    w, ws = make_weights(ModelShape("gate_up", 2 * inter, k), 2, "cuda")
+    down, down_s = make_weights(ModelShape("down", 256, inter), 5, "cuda")
+    x = make_activations(m, k, 2).cuda()
+    takes = offset == 0 and not fp8.dispatch_name(m, 2 * inter, k).startswith("stream")
+    expect = fp8.mlp_forward_mi355x_fp8(x, w, ws, down, down_s)
+    held = torch.empty(w.numel() + 16, device="cuda", dtype=torch.uint8)
+    held[offset:offset + w.numel()] = w.view(torch.uint8).flatten()
+    w = held[offset:offset + w.numel()].view(torch.float8_e4m3fn).view(2 * inter, k)
+    seen = []
+    quantize = fp8.quantize_mi355x_fp8_activation
+    monkeypatch.setattr(fp8, "quantize_mi355x_fp8_activation",
+                        lambda t, **kw: (seen.append(tuple(t.shape)), quantize(t, **kw))[1])
+    assert bitwise_equal(fp8.mlp_forward_mi355x_fp8(x, w, ws, down, down_s), expect)
+    assert seen == ([(m, k), (m, inter)] if takes else [])
+
+
 def test_silu_over_every_bf16_gate():
     """silu(g) for all 65536 bf16 gates (up = 1): the short form within half a bf16 place of the
     exact value plus its own fp32 error (below 2^-20, so 2^-10 of the half place is ample); the
