@@ -7,6 +7,9 @@
 // the wrapper goes on as before (it holds the error messages, the copies of strided operands and
 // the growing of the workspace), so what is accepted and what is refused is decided there.
 //
+// The interpreter lock is held over the launches: threads that share a stream share its workspace,
+// and their quantizer and GEMM launches must not interleave.
+//
 // No state lives here but the per-device architecture check (device properties do not change).
 // The workspace is the caller's: `buffers` is the wrapper's {(device, stream): byte tensor} dict.
 #include <ATen/ATen.h>
@@ -17,6 +20,8 @@
 
 #include <atomic>
 #include <cstring>
+#include <stdexcept>
+#include <string>
 
 #include "../../include/mi355x_fp8.h"
 
@@ -77,6 +82,11 @@ py::object linear(const at::Tensor& x, const at::Tensor& w, const at::Tensor& ws
       static_cast<const uint8_t*>(w.data_ptr()), w.stride(0), static_cast<const float*>(ws.data_ptr()), ws.stride(0),
       ws.stride(1), n, out.data_ptr(), dtype_code(out_type), n, workspace.data_ptr(), bytes, MI355X_FP8_CONFIG_AUTO,
       stream);
+  // A failed launch is reported here: running the call again in the wrapper could succeed and hide
+  // it.  Any other status is a refusal, which the wrapper words.
+  if (status == MI355X_FP8_ERR_LAUNCH)
+    throw std::runtime_error("libmi355x_fp8: " + std::string(mi355x_fp8_status_string(status)) + " (status " +
+                             std::to_string(status) + ")");
   if (status != MI355X_FP8_OK) return py::none();
   if (x.dim() > 2) {
     std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());

@@ -1,11 +1,14 @@
 """The native common case of mi355x_fp8_linear against the wrapper's own path, over the forms it
 accepts and the ones it leaves to the wrapper."""
 
+import ctypes
+
 import pytest
 import torch
 
 from minillm_amd import _lib
 from minillm_amd import mi355x_fp8 as fp8
+from minillm_amd.build import LIB_PATH
 from minillm_amd.validation import ModelShape, bitwise_equal, make_activations, make_weights
 
 pytestmark = pytest.mark.gpu
@@ -78,3 +81,19 @@ def test_native_on_other_streams_and_after_clear():
         assert bitwise_equal(out, ref[:m])
     fp8._workspace.clear()
     assert bitwise_equal(fp8.mi355x_fp8_linear(x, w, ws, [128, 128]), ref)
+
+
+def test_native_reports_a_failed_launch(monkeypatch):
+    """A HIP error that the launch check finds (here one left behind by a refused host call) is
+    raised by the native call as by the wrapper, once, and not covered up by a second launch."""
+
+    x, w, ws = _operands(33)
+    ref = fp8.mi355x_fp8_linear(x, w, ws, [128, 128])
+    torch.cuda.synchronize()
+    hip_set_device = ctypes.CDLL(LIB_PATH).hipSetDevice
+    args = (x, w, ws, [128, 128])
+    for call in (lambda: _wrapper(monkeypatch, *args), lambda: fp8.mi355x_fp8_linear(*args)):
+        assert hip_set_device(4096) != 0
+        with pytest.raises(RuntimeError, match=r"launch failed \(status 4\)"):
+            call()
+        assert bitwise_equal(call(), ref)
