@@ -906,14 +906,23 @@ PrefillChoice choose_prefill(int64_t M, int64_t N, int64_t cus, bool rows256_ok)
 // 41.3; 32 x 19456 x 2560 64x128 15.9 / 64x96 13.7, at 64 rows 19.5 / 15.3; 128 x 19456 x 2560
 // 128x128 21.4 / 128x96 18.7; 200 x 6144 x 2560 128x64 16 / 64x96 11.1.  Neighbours in the order
 // differ by little (700 x 2560 x 9728: 128x64 30.2, 96x96 31.1, 128x96 36.0, 96x128 36.0).
-constexpr PrefillChoice kSingleWave[] = {{64, 64},  {96, 64},  {64, 96},  {128, 64}, {96, 96},
-                                         {64, 128}, {96, 128}, {128, 96}, {128, 128}};
+// 64x128 and 96x96 tiles read as many operand rows a K group and cost alike, so of those two the
+// one with more tiles, whose CUs each hold less (us, 64x128 / 96x96): qkv at 288 rows, 240 / 192
+// tiles, 13.7 / 14.6, at 300 rows, 240 / 256 tiles, 14.0 / 12.4; 192 x 9728 x 2560, 228 / 204
+// tiles, 15.0 / 15.5.
+constexpr PrefillChoice kSingleWave[] = {{64, 64},  {96, 64},  {64, 96},  {128, 64}, {64, 128},
+                                         {96, 96},  {96, 128}, {128, 96}, {128, 128}};
 
 PrefillChoice prefill_tile(int64_t M, int64_t N, int64_t cus, bool rows256_ok) {
   const PrefillChoice c = choose_prefill(M, N, cus, rows256_ok);
   if (c.rows > 128 || cdiv(M, c.rows) * cdiv(N, c.bn) > cus) return c;
-  for (const PrefillChoice& t : kSingleWave)
-    if (cdiv(M, t.rows) * cdiv(N, t.bn) <= cus) return t;
+  const auto tiles = [&](const PrefillChoice& t) { return cdiv(M, t.rows) * cdiv(N, t.bn); };
+  for (const PrefillChoice& t : kSingleWave) {
+    if (tiles(t) > cus) continue;
+    constexpr PrefillChoice kSquare{96, 96};
+    if (t.rows == 64 && t.bn == 128 && tiles(kSquare) > tiles(t) && tiles(kSquare) <= cus) return kSquare;
+    return t;
+  }
   return c;
 }
 }  // namespace

@@ -194,6 +194,10 @@ def test_dispatch_choice_names_the_stream_kernel_then_the_prefill_tiles():
     assert fp8.dispatch_name(2048, 6144, 2000) == "tile 128x128"
     assert fp8.dispatch_name(536, 2560, 4000) == "tile 96x64"
     assert fp8.dispatch_name(2048, 6144, 2001) == "tile 128x128"
+    # 64x128 or 96x96, whichever has more tiles.
+    assert [fp8.dispatch_name(m, 6144, 2560) for m in (257, 288, 289, 320)] == [
+        "tile 64x128", "tile 64x128", "tile 96x96", "tile 96x96"]
+    assert [fp8.dispatch_name(m, 9728, 2560) for m in (144, 192)] == ["tile 64x128", "tile 64x128"]
     lib = _lib.load()
     a, b, c = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     assert lib.mi355x_fp8_dispatch_choice(0, 2560, 2560, 256, ctypes.byref(a), ctypes.byref(b),
