@@ -516,8 +516,15 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
     __syncthreads();
     constexpr int C = (SILU ? BN / 2 : BN) / 8;  // 16-byte pieces per row
     const int64_t n_end = SILU ? half : N;
+    constexpr int kPieces = G::kRows * C;
+    constexpr int kPasses = (kPieces + kDmaThreads - 1) / kDmaThreads;
+    // A constant trip count, so that the passes unroll and the indices are formed once: formed in
+    // every pass, the 160-wide single wave issued 0.9 % more VALU instructions over the whole kernel
+    // and the two-per-CU 128x128 form took 38.0 instead of 37.8 us (2048 x 2560 x 4096).
 #pragma unroll
-    for (int idx = tid; idx < G::kRows * C; idx += kDmaThreads) {
+    for (int it = 0; it < kPasses; ++it) {
+      const int idx = tid + it * kDmaThreads;
+      if (kPieces % kDmaThreads != 0 && idx >= kPieces) break;
       const int row = idx / C, c = idx - (idx / C) * C;
       const int64_t m = m0 + row, n = n0 + 8 * c;
       const uint16_t* reg_r = reinterpret_cast<const uint16_t*>(row < kHalf ? stage0 : stage1);
