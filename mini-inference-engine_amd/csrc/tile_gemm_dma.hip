@@ -11,7 +11,7 @@
 //
 // What differs is the feed: global memory goes straight into LDS with
 // global_load_lds_dwordx4 (no register staging, no ds_write), through a ring of STAGES
-// stages (2 when two workgroups share a CU, else 4, or 3 at width 160).  Each stage holds the W tile (BN rows x 128 B), the activation tile
+// stages (2 when two workgroups share a CU, else 4, or 3 at width 160 and over few K groups).  Each stage holds the W tile (BN rows x 128 B), the activation tile
 // (128 x 128 B) and the 128 activation scales of its K group.  A 64-lane DMA instruction fills 1 KiB of LDS
 // linearly (lane i -> byte 16 i), i.e. 8 rows of 8 16-byte chunks; the XOR swizzle
 // (physical chunk p of row r holds logical chunk p ^ (r & 7)) is applied by choosing each
@@ -26,7 +26,7 @@
 // step, which read the fragments of its first MFMAs during the previous step only (us, weights
 // from HBM): N = 2560 at 536 rows K = 4096 17.1 -> 14.3, K = 9728 32.6 -> 28.0.
 // Two workgroups per CU (two stages, k_step; also 256 registers at most): the two hide each
-// other's waits.  The 160-wide single waves (three stages) keep this step too: twenty MFMAs a step
+// other's waits.  Three stages take this step too.  The 160-wide single waves keep it at any depth: twenty MFMAs a step
 // hide most of the reads already, and the other step measured 29.5 against 28.5 us (N = 2560, K =
 // 4096 at 2048 rows, weights from HBM; K = 9728 the same).  A K step reads the fragments of its first MFMAs during the previous step, each
 // later weight fragment while the MFMAs of the one before run, and the barrier sits between the
@@ -58,6 +58,8 @@ namespace {
 constexpr int kDmaThreads = 256;
 constexpr int kStagesFew = 4;   // ring depth when the tiles do not exceed the CUs
 constexpr int kStagesFew160 = 3;  // the same for the 160-wide tiles, with the two-part k_step
+constexpr int kStagesShallow = 3;  // and for the 128x128 and 64-row tiles over few K groups
+constexpr int kShallowGroups128 = 28, kShallowGroups64 = 4;  // few: up to this many (launch_tile_dma)
 constexpr int kStagesMany = 2;  // otherwise (two workgroups per CU)
 constexpr int kTileRows = 128;                          // activation rows per tile
 constexpr int kMaxBN = 160;                             // widest W tile (columns of the output tile)
@@ -591,6 +593,12 @@ int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_s
   // 536 rows).  64x64 tiles have room for two workgroups of four stages.
   const bool few = tiles_m * tiles_n <= device_cus();
   if (!few && (rows == 96 || bn == 96)) return MI355X_FP8_ERR_INVALID;
+  // The four-stage ring fills and, past the end of K, refills one stage more than the three-stage
+  // one, 0.2-0.5 us a launch that its shorter steps have to earn back.  Where the lines lie
+  // (us, four stages with reg_step / three with k_step, one wave of 247 tiles): 128x128 at K = 512 7.2 /
+  // 6.8, 1024 8.9 / 8.6, 2560 16.7 / 16.3, 3584 20.8 / 20.7, 4096 22.4 / 22.9; 64x128 at K = 256 5.1 /
+  // 4.8, 512 5.6 / 5.5, 1024 6.6 / 6.6, 2560 10.2 / 10.6; 64x64 at K = 256 4.2 / 3.9, 1536 6.4 / 6.6.
+  const bool shallow = few && (K + kGroup - 1) / kGroup <= (rows == 128 ? kShallowGroups128 : kShallowGroups64);
 #define MI355X_DMA_ARGS q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, o, ldo, M, N, (K + kGroup - 1) / kGroup, tiles_m, tiles_n, vec_out, tail
 #define MI355X_DMA_LAUNCH_T(ST, BN, T, J, KT, SI) \
   tile_gemm_dma_kernel<ST, BN, T, J, KT, SI><<<grid, kDmaThreads, 0, stream>>>(MI355X_DMA_ARGS)
@@ -605,8 +613,10 @@ int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_s
     else MI355X_DMA_LAUNCH(kStagesMany, BN, J);             \
   } while (0)
   if (rows == 64) {
-    if (bn == 64) MI355X_DMA_LAUNCH(kStagesFew, 64, 2);
+    if (bn == 64 && shallow) MI355X_DMA_LAUNCH(kStagesShallow, 64, 2);
+    else if (bn == 64) MI355X_DMA_LAUNCH(kStagesFew, 64, 2);
     else if (bn == 96) MI355X_DMA_LAUNCH(kStagesFew, 96, 2);
+    else if (shallow) MI355X_DMA_LAUNCH(kStagesShallow, 128, 2);
     else MI355X_DMA_ROWS(128, 2);
   } else if (rows == 96) {
     if (bn == 64) MI355X_DMA_LAUNCH(kStagesFew, 64, 3);
@@ -617,6 +627,7 @@ int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_s
     else if (bn == 160) MI355X_DMA_LAUNCH(kStagesMany, 160, 4);
     else if (bn == 96) MI355X_DMA_LAUNCH(kStagesFew, 96, 4);
     else if (bn == 64) MI355X_DMA_ROWS(64, 4);
+    else if (shallow) MI355X_DMA_LAUNCH(kStagesShallow, 128, 4);
     else MI355X_DMA_ROWS(128, 4);
   }
 #undef MI355X_DMA_ROWS

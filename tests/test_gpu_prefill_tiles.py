@@ -42,6 +42,28 @@ def test_linear_equals_register_kernel(m, n, k, dtype):
     assert bitwise_equal(got, ref), bit_mismatch_details(got, ref)
 
 
+@pytest.mark.parametrize("m,n,tile,depths", [
+    (96, 320, "64x64", (128, 256, 384, 512, 640, 16, 272, 400)), (257, 6144, "64x128", (128, 384, 512, 640, 208, 528)),
+    (600, 6144, "128x128", (128, 256, 384, 512, 3584, 3712, 144, 3472)),
+])
+def test_three_stage_ring_equals_register_kernel(m, n, tile, depths):
+    """Single-wave tiles over few K groups: one group, every remainder of the three-stage ring and
+    both sides of the depth where the ring gets its fourth stage; whole and ending in a tail; the
+    plain output and, where K is whole, SiLU*up."""
+
+    for k in depths:
+        assert fp8.dispatch_name(m, n, k) == f"tile {tile}"
+        x = make_activations(m, k, 13).cuda()
+        w, ws = make_weights(ModelShape("shallow", n, k), 13, "cuda")
+        got, ref = fp8.mi355x_fp8_linear(x, w, ws, [128, 128]), _reference(x, w, ws, torch.bfloat16)
+        assert bitwise_equal(got, ref), (k, bit_mismatch_details(got, ref))
+        if k % 128 == 0:
+            q, s = fp8.quantize_mi355x_fp8_activation(x, scale_layout="kgroup")
+            h = fp8.silu_mul_quant_mi355x_fp8(ref[:, :n // 2], ref[:, n // 2:], return_intermediate=True)[0]
+            got = fp8._gemm_silu(q, s, w, ws)
+            assert bitwise_equal(got, h), (k, bit_mismatch_details(got, h))
+
+
 @pytest.mark.parametrize("k", [144, 400])
 def test_k_tail_keeps_a_nan_code_in_its_own_column(k):
     """The tail's out-of-range weight chunks read other chunks of the same row: a NaN code there
