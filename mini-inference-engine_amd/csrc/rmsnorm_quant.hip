@@ -25,16 +25,17 @@
 //
 // Layout: a workgroup of 4 waves holds 4 / wpr rows, each row spread over wpr waves (4 for
 // up to 512 rows, else 2; the reduction order does not depend on wpr).  The
-// norm weight and the rows are read once into LDS (rows up to 16128 wide).  Virtual thread
-// t of the reduction lives in lane t % 64 of the row's wave (t / 64) % wpr (reductions of 32
-// threads, 16 rows and more: in every wave, two lanes each), so folds with
-// h >= 64 wpr stay inside a lane, folds between 64 and 64 wpr go through LDS, and the rest
-// are shuffles.  The second pass normalizes and quantizes one 128-wide group per 16-lane
-// slice, 8 elements per lane.
+// norm weight and the rows are read once into LDS (rows up to 16128 wide).  A reduction of 32
+// virtual threads (16 rows and more, or rows narrower than 256) runs whole in every wave, two
+// lanes a thread.  A wider one (64 to 512 threads) has thread t in lane t % 64 of wave
+// (t / 64) % 4: the fold with h = 256 stays inside a lane, those with h = 128 and 64 go through
+// LDS.  The rest are lane swaps and DPP moves.  The second pass normalizes and quantizes one
+// 128-wide group per 16-lane slice, 8 elements per lane.
 // A latency chain (load, reduce, normalize, store) on few waves per SIMD, not bandwidth, bounds it:
 // with every wave of a row forming the whole sum from reads issued ahead, no redundant loads and
 // the quantizer's short divisions, 32 rows x 2560 with the residual went from 6.3 to 4.8 us, 2048
-// rows from 13.1 to 11.5 (3.2 TB/s).
+// rows from 13.1 to 11.5 (3.2 TB/s); below 16 rows, without slots that no thread count fills, 1 row
+// from 4.6 to 3.9 and 8 rows from 4.6 to 4.4 (back to back in a graph).
 // HBM traffic per row: 2K bytes in (4K with the residual), K + 4K/128 out (+2K for the
 // residual sum).
 #include "fp8_abi_internal.h"
@@ -134,15 +135,12 @@ __global__ __launch_bounds__(64 * kRnqWavesPerBlock) void rmsnorm_quant_kernel(
   }
   __syncthreads();  // the weight and the rows are in LDS
 
-
   // ---- pass 1: sum of squares in the reference's order ----------------------------
-  // Virtual thread t lives in lane t % 64 of wave (t / 64) % wpr, as its slot j = t / (64 wpr).
-  // Waves past the last row run it on whatever their LDS holds and discard the result: every
-  // wave has to reach the barrier below.
+  // Waves past the last row run it on whatever their LDS holds and discard the result.
   const int64_t nvec = K / 4;
   float ssum;
   if (bw == 32) {
-    // 16 rows and more of a wide row: 32 virtual threads.  Every wave of the row forms the whole
+    // 32 virtual threads.  Every wave of the row forms the whole
     // sum, so nothing is exchanged between waves; lane l holds accumulators 2 h and 2 h + 1 (h =
     // l / 32) of thread l % 32, whose vectors are read kAhead at a time ahead of the chain.
     constexpr int kAhead = 10;
@@ -167,12 +165,14 @@ __global__ __launch_bounds__(64 * kRnqWavesPerBlock) void rmsnorm_quant_kernel(
     ssum = tree_sum32(__fadd_rn(__fadd_rn(__fadd_rn(a0, a1), upper(a0)), upper(a1)));
     if (!live) return;  // no barrier follows
   } else {
-    const int span = 64 * wpr;  // virtual threads per slot
-    float part[8];              // bw <= 512: at most 8 slots per lane
+    // Fewer than 16 rows: 64 to 512 virtual threads over the row's four waves (wpr = 4, one row a
+    // workgroup, all of them live).
+    constexpr int kSpan = 256;
+    float part[2];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < 2; ++j) {
       part[j] = 0.0f;
-      const int t = rl + span * j;
+      const int t = rl + kSpan * j;
       if (t >= bw) continue;
       float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
       for (int64_t v = t; v < nvec; v += bw) {
@@ -184,41 +184,21 @@ __global__ __launch_bounds__(64 * kRnqWavesPerBlock) void rmsnorm_quant_kernel(
       }
       part[j] = __fadd_rn(__fadd_rn(__fadd_rn(a[0], a[1]), a[2]), a[3]);
     }
-    // Folds with h >= 64 wpr: slots j and j + h / (64 wpr) of the same lane.
-    for (int h = bw / 2; h >= span; h >>= 1) {
-      const int hj = h / span;
+    // The fold with h = 256: the two slots of a lane.
+    ssum = bw == 2 * kSpan ? __fadd_rn(part[0], part[1]) : part[0];
+    // Folds with h = 128 and 64: the same lane of waves sub and sub + h / 64, through LDS.
+    red[rl] = ssum;
+    __syncthreads();
+    const int nsub = bw >= kSpan ? 4 : bw / 64;
+    float v[4];
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (j < hj) part[j] = __fadd_rn(part[j], part[j + hj]);
-    }
-    // Folds with 64 <= h < 64 wpr: the same lane of waves sub and sub + h / 64, through LDS.
-    ssum = part[0];
-    if (wpr > 1) {
-      red[rl] = ssum;
-      __syncthreads();
-      const int nsub = bw >= span ? wpr : (bw >= 64 ? bw / 64 : 1);
-      float v[4];
+    for (int i = 0; i < 4; ++i) v[i] = i < nsub ? red[i * 64 + lane] : 0.0f;
+    for (int h = nsub / 2; h >= 1; h >>= 1) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = i < nsub ? red[i * 64 + lane] : 0.0f;
-      for (int h = nsub / 2; h >= 1; h >>= 1) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-          if (i < h) v[i] = __fadd_rn(v[i], v[i + h]);
-      }
-      ssum = v[0];
+      for (int i = 0; i < 2; ++i)
+        if (i < h) v[i] = __fadd_rn(v[i], v[i + h]);
     }
-    if (!live) return;  // no barrier follows
-    // Folds with h < 64: lane l adds lane l + h (tree_sum64: lane swaps and DPP; a reduction
-    // narrower than a wave keeps the shuffles).
-    if (bw >= 64) {
-      ssum = tree_sum64(ssum);
-    } else {
-      for (int h = bw / 2; h >= 1; h >>= 1) {
-        const float other = __shfl_down(ssum, h, 64);
-        if (lane < h) ssum = __fadd_rn(ssum, other);
-      }
-      ssum = __shfl(ssum, 0, 64);
-    }
+    ssum = tree_sum64(v[0]);  // folds with h < 64
   }
   const float var = __fmul_rn(ssum, inv_k);
   const float inv = rsqrt_rn(__fadd_rn(var, eps));
@@ -317,7 +297,7 @@ int launch_rmsnorm_quant(const uint16_t* x, int64_t sxm, const uint16_t* res, in
   const int vec = K % 8 == 0 && sxm % 8 == 0 && aligned16(x) && aligned16(weight) && aligned16(y ? y : x) &&
                   (ldq % 8) == 0 && (reinterpret_cast<uintptr_t>(q) % 8) == 0 &&
                   (res == nullptr || (ldr % 8 == 0 && ldro % 8 == 0 && aligned16(res) && aligned16(res_out)));
-  const int bw = rmsnorm_block_width(M, K);
+  const int bw = rmsnorm_block_width(M, K);  // 32 from 16 rows up or below K = 256, else 64 to 512
   const float inv_k = 1.0f / static_cast<float>(K);
   const dim3 grid(static_cast<unsigned>(blocks));
   const size_t lds = static_cast<size_t>(rows + 1) * row_bytes + static_cast<size_t>(rows) * 64 * wpr * 4;
