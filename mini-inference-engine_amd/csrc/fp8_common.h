@@ -81,8 +81,8 @@ __device__ __forceinline__ float round_bf16(float f) {
 
 // bf16(g / (1 + exp(-g))) of N bf16 gate values, in place.  The function depends on the 16 bits of
 // g alone, so the short form below (the hardware exp2 and reciprocal, one Newton step on the
-// reciprocal) was compared with the IEEE division and expf over all 65536 of them: equal bits
-// wherever g > -86.  Below that, where 1 + exp(-g) nears the largest float and its reciprocal the
+// reciprocal) is compared with the IEEE division and expf over all 65536 of them
+// (tests/test_short_forms.py): equal bits wherever g > -86.  Below that, where 1 + exp(-g) nears the largest float and its reciprocal the
 // denormals, and for a NaN, the group takes the long form.  About 13 issue slots an element
 // instead of 32: the SiLU*up quantizer at 2048 x 9728 33.4 -> 25.8 us.
 template <int N>
@@ -133,8 +133,9 @@ __device__ __forceinline__ void store8_cols(uint16_t* dst, uint4 v, int64_t n, i
 
 // 1 / sqrt(v) rounded once to fp32, as through double square root and division: the hardware's
 // double reciprocal square root and one third-order Newton step, a chain of 6 operations instead of
-// some 25 in front of everything a norm still has to do.  Compared with (float)(1.0 / sqrt((double)v))
-// over every positive finite fp32 v: equal bits.  Zero, infinity and NaN take that form.
+// some 25 in front of everything a norm still has to do.  The bits of (float)(1.0 / sqrt((double)v)) for
+// every positive finite fp32 v from any estimate within the 2^-23 that the instruction states
+// (tests/c/short_forms_check.c).  Zero, infinity and NaN take that form.
 __device__ __forceinline__ float rsqrt_rn(float v) {
   const double d = static_cast<double>(v);
   if (!(v > 0.0f && v < __builtin_inff())) return static_cast<float>(1.0 / sqrt(d));
@@ -164,9 +165,9 @@ __device__ __forceinline__ float div_by_scale(float t, float den, float r) {
 
 // amax / 448, correctly rounded, by div_by_scale's remainder correction with a constant reciprocal
 // (an infinity stays one), and 1 / den for a finite den >= 1e-12, by one Newton step on the
-// hardware reciprocal: 5 and 3 issue slots instead of the 11 and 10 of the divisions.  Both were
-// compared with IEEE division over every amax that a group of bf16 or fp16 values can have (and the
-// den it gives): equal bits.
+// hardware reciprocal: 5 and 3 issue slots instead of the 11 and 10 of the divisions.  The bits of
+// IEEE division over every finite amax of bf16 and fp16 values (and the den it gives), from any reciprocal
+// within 2 ulp (tests/c/short_forms_check.c; on the GPU tests/test_short_forms.py).
 __device__ __forceinline__ float scale_of(float amax) {
   constexpr float r = 1.0f / 448.0f;
   const float q0 = amax * r;

@@ -3,7 +3,8 @@
 //
 // For every amax (positive finite value of the 16-bit format) and every t of the format
 // with |t| <= amax (the elements of a group are bounded by its amax) or t NaN:
-//   den = max(amax / 448, 1e-12), r = 1 / den            (IEEE, correctly rounded)
+//   den = max(amax / 448, 1e-12), r = 1 / den            (IEEE, correctly rounded; the bits of the
+//                                                         device's scale_of and recip_den: short_forms_check.c)
 //   q0 = t * r, rem = fma(-q0, den, t), q = copysign(fma(rem, r, q0), t)
 // must equal t / den bitwise wherever |t / den| >= 2^-12; below that (every such quotient
 // becomes an e4m3 zero) only the sign has to match, and NaN must stay NaN with t's sign.
