@@ -11,7 +11,8 @@
 //
 // What differs is the feed: global memory goes straight into LDS with
 // global_load_lds_dwordx4 (no register staging, no ds_write), through a ring of STAGES
-// stages (2 when two workgroups share a CU, else 4, or 3 at width 160 and over few K groups).  Each stage holds the W tile (BN rows x 128 B), the activation tile
+// stages (2 when two workgroups share a CU, else 4, or 3 at width 160 and over few K groups, or 6 for
+// 64x64 tiles over many).  Each stage holds the W tile (BN rows x 128 B), the activation tile
 // (128 x 128 B) and the 128 activation scales of its K group.  A 64-lane DMA instruction fills 1 KiB of LDS
 // linearly (lane i -> byte 16 i), i.e. 8 rows of 8 16-byte chunks; the XOR swizzle
 // (physical chunk p of row r holds logical chunk p ^ (r & 7)) is applied by choosing each
@@ -60,6 +61,8 @@ constexpr int kStagesFew = 4;   // ring depth when the tiles do not exceed the C
 constexpr int kStagesFew160 = 3;  // the same for the 160-wide tiles, with the two-part k_step
 constexpr int kStagesShallow = 3;  // and for the 128x128 and 64-row tiles over few K groups
 constexpr int kShallowGroups128 = 28, kShallowGroups64 = 4;  // few: up to this many (launch_tile_dma)
+constexpr int kStagesDeep = 6;     // and for 64x64 tiles over many K groups whose last row tile is part empty
+constexpr int kDeepGroups = 24, kDeepRows = 40;  // from this many groups, up to this many rows in it
 constexpr int kStagesMany = 2;  // otherwise (two workgroups per CU)
 constexpr int kTileRows = 128;                          // activation rows per tile
 constexpr int kMaxBN = 160;                             // widest W tile (columns of the output tile)
@@ -449,11 +452,15 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
 #pragma unroll
     for (int j = 0; j < J; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
-  static_assert(STAGES >= 2 && STAGES <= 4, "stages");
+  static_assert((STAGES >= 2 && STAGES <= 4) || STAGES == 6, "stages");
   issue_stage<BN, 0, J, KTAIL>(ring, src, 0, KB, as_sk, wave);
   issue_stage<BN, 1, J, KTAIL>(ring, src, KB > 1 ? 1 : KB - 1, KB, as_sk, wave);
   if constexpr (STAGES >= 3) issue_stage<BN, 2, J, KTAIL>(ring, src, KB > 2 ? 2 : KB - 1, KB, as_sk, wave);
   if constexpr (STAGES >= 4) issue_stage<BN, 3, J, KTAIL>(ring, src, KB > 3 ? 3 : KB - 1, KB, as_sk, wave);
+  if constexpr (STAGES == 6) {
+    issue_stage<BN, 4, J, KTAIL>(ring, src, KB > 4 ? 4 : KB - 1, KB, as_sk, wave);
+    issue_stage<BN, 5, J, KTAIL>(ring, src, KB > 5 ? 5 : KB - 1, KB, as_sk, wave);
+  }
   wait_vm_lgkm0<G::kDmaPerStage * (STAGES - 1)>();
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
@@ -486,11 +493,19 @@ __global__ __launch_bounds__(kDmaThreads, STAGES == 2 ? 2 : 1) void tile_gemm_dm
       MI355X_KSTEP(1, f1, f0, kb + 1);
       MI355X_KSTEP(2, f0, f1, kb + 2);
       MI355X_KSTEP(3, f1, f0, kb + 3);
+      if constexpr (STAGES == 6) {
+        MI355X_KSTEP(4, f0, f1, kb + 4);
+        MI355X_KSTEP(5, f1, f0, kb + 5);
+      }
     }
     // The last KB % STAGES groups.
     if (kb < KB) MI355X_KSTEP(0, f0, f1, kb);
     if (kb + 1 < KB) MI355X_KSTEP(1, f1, f0, kb + 1);
     if (kb + 2 < KB) MI355X_KSTEP(2, f0, f1, kb + 2);
+    if constexpr (STAGES == 6) {
+      if (kb + 3 < KB) MI355X_KSTEP(3, f1, f0, kb + 3);
+      if (kb + 4 < KB) MI355X_KSTEP(4, f0, f1, kb + 4);
+    }
 #undef MI355X_KSTEP
   }
   wait_vm_lgkm0<0>();  // no DMA may still target LDS when the workgroup ends
@@ -589,7 +604,7 @@ int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_s
   if (silu && (vec_out != 2 || out_dtype != kBF16 || tail != 0)) return MI355X_FP8_ERR_INVALID;
   // Two stages (76 KiB, room for the 160-wide W tile) let two workgroups share a CU.  When the
   // tiles do not fill the CUs anyway, four stages (one workgroup per CU) keep more K groups in
-  // flight; six, where they fit, measured the same (28.0 and 28.3 us for N = 2560, K = 9728 at
+  // flight; six, where they fit, measured the same at 128x64 (28.0 and 28.3 us for N = 2560, K = 9728 at
   // 536 rows).  64x64 tiles have room for two workgroups of four stages.
   const bool few = tiles_m * tiles_n <= device_cus();
   if (!few && (rows == 96 || bn == 96)) return MI355X_FP8_ERR_INVALID;
@@ -598,8 +613,19 @@ int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_s
   // (us, four stages with reg_step / three with k_step, one wave of 247 tiles): 128x128 at K = 512 7.2 /
   // 6.8, 1024 8.9 / 8.6, 2560 16.7 / 16.3, 3584 20.8 / 20.7, 4096 22.4 / 22.9; 64x128 at K = 256 5.1 /
   // 4.8, 512 5.6 / 5.5, 1024 6.6 / 6.6, 2560 10.2 / 10.6; 64x64 at K = 256 4.2 / 3.9, 1536 6.4 / 6.6.
-  const bool shallow = few && (K + kGroup - 1) / kGroup <= (rows == 128 ? kShallowGroups128 : kShallowGroups64);
-#define MI355X_DMA_ARGS q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, o, ldo, M, N, (K + kGroup - 1) / kGroup, tiles_m, tiles_n, vec_out, tail
+  const int64_t groups = (K + kGroup - 1) / kGroup;
+  const bool shallow = few && groups <= (rows == 128 ? kShallowGroups128 : kShallowGroups64);
+  // 64x64 tiles, whose steps are the shortest: reg_step has half a step less in flight than k_step
+  // had in as many stages, and lost up to 1.5 % to it where tiles of a part-empty last row tile (whose
+  // rows past M read one line) run ahead and wait on HBM.  Six stages take that back and more.  us,
+  // four stages with k_step / four / six with reg_step, N = 2560, weights from HBM: K = 9728 at 65 rows
+  // 23.1 / 23.3 / 19.4, 84 23.2 / 23.4 / 20.5, 200 23.4 / 23.5 / 20.0, 104 24.0 / 24.1 / 23.5; K = 3072 at
+  // 70 rows 9.8 / 9.9 / 9.1, 104 10.2 / 10.1 / 10.1.  With a fuller last tile or fewer groups the longer
+  // fill costs 0.1-0.4 us: K = 9728 at 112 rows 24.6 / 24.5 / 24.7, 128 25.7 / 25.6 / 25.9; K = 2048 at 100
+  // rows 7.9 / 7.9 / 8.0, N = 4096, K = 2560 at 102 rows 9.35 / 9.34 / 9.66.
+  const int64_t last_rows = (M - 1) % 64 + 1;
+  const bool deep = few && groups >= kDeepGroups && last_rows <= kDeepRows;
+#define MI355X_DMA_ARGS q, ldq, as, as_sk, w, ldw, ws, ws_sn, ws_sk, o, ldo, M, N, groups, tiles_m, tiles_n, vec_out, tail
 #define MI355X_DMA_LAUNCH_T(ST, BN, T, J, KT, SI) \
   tile_gemm_dma_kernel<ST, BN, T, J, KT, SI><<<grid, kDmaThreads, 0, stream>>>(MI355X_DMA_ARGS)
 #define MI355X_DMA_LAUNCH_K(ST, BN, J, KT)                                       \
@@ -614,6 +640,7 @@ int launch_tile_dma(const uint8_t* q, int64_t ldq, const float* as, int64_t as_s
   } while (0)
   if (rows == 64) {
     if (bn == 64 && shallow) MI355X_DMA_LAUNCH(kStagesShallow, 64, 2);
+    else if (bn == 64 && deep) MI355X_DMA_LAUNCH(kStagesDeep, 64, 2);
     else if (bn == 64) MI355X_DMA_LAUNCH(kStagesFew, 64, 2);
     else if (bn == 96) MI355X_DMA_LAUNCH(kStagesFew, 96, 2);
     else if (shallow) MI355X_DMA_LAUNCH(kStagesShallow, 128, 2);

@@ -64,6 +64,26 @@ def test_three_stage_ring_equals_register_kernel(m, n, tile, depths):
             assert bitwise_equal(got, h), (k, bit_mismatch_details(got, h))
 
 
+@pytest.mark.parametrize("m", [65, 104, 105, 128])
+def test_six_stage_ring_equals_register_kernel(m):
+    """64x64 tiles over many K groups, with a last row tile on both sides of the six-stage ring's
+    bound and a full one: every remainder of the ring and the depth below its first, whole and ending
+    in a tail; the plain output and, where K is whole, SiLU*up."""
+
+    n = 320
+    for k in (2944, 3072, 3200, 3328, 3456, 3584, 3712, 2960, 3184, 3440):
+        assert fp8.dispatch_name(m, n, k) == "tile 64x64"
+        x = make_activations(m, k, 17).cuda()
+        w, ws = make_weights(ModelShape("deep", n, k), 17, "cuda")
+        got, ref = fp8.mi355x_fp8_linear(x, w, ws, [128, 128]), _reference(x, w, ws, torch.bfloat16)
+        assert bitwise_equal(got, ref), (k, bit_mismatch_details(got, ref))
+        if k % 128 == 0:
+            q, s = fp8.quantize_mi355x_fp8_activation(x, scale_layout="kgroup")
+            h = fp8.silu_mul_quant_mi355x_fp8(ref[:, :n // 2], ref[:, n // 2:], return_intermediate=True)[0]
+            got = fp8._gemm_silu(q, s, w, ws)
+            assert bitwise_equal(got, h), (k, bit_mismatch_details(got, h))
+
+
 @pytest.mark.parametrize("k", [144, 400])
 def test_k_tail_keeps_a_nan_code_in_its_own_column(k):
     """The tail's out-of-range weight chunks read other chunks of the same row: a NaN code there

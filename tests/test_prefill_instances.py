@@ -17,7 +17,7 @@ TILE128 = next(c for c in fp8.GEMM_CONFIGS if c.name == "tile128")
 # (rows, width, ring) -> (M, N, K groups).  The ring: its stages where the tiles fit one per CU,
 # "many" where they do not; the 192- and 256-row tiles have one ring each.
 CASES = {
-    (64, 64, 3): (65, 96, 4), (64, 64, 4): (65, 96, 5), (64, 64, "many"): (17, 16800, 5),
+    (64, 64, 3): (65, 96, 4), (64, 64, 4): (65, 96, 5), (64, 64, 6): (65, 96, 29), (64, 64, "many"): (17, 16800, 5),
     (64, 96, 4): (17, 17632, 5),
     (64, 128, 3): (17, 24832, 4), (64, 128, 4): (17, 24832, 5), (64, 128, "many"): (17, 33280, 5),
     (96, 64, 4): (65, 8480, 6), (96, 96, 4): (65, 16800, 7), (96, 128, 4): (65, 24832, 5),
@@ -50,6 +50,8 @@ def _instance(m, n, k):
     if -(-m // tile[0]) * -(-n // tile[1]) > CUS:
         return (*tile, "many")
     groups = -(-k // 128)
+    if tile == (64, 64) and groups >= 24 and 1 <= m % 64 <= 40:
+        return (*tile, 6)
     three = tile == (128, 160) or (tile == (128, 128) and groups <= 28) or (tile in ((64, 64), (64, 128)) and groups <= 4)
     return (*tile, 3 if three else 4)
 
