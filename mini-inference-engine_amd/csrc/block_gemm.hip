@@ -850,8 +850,17 @@ int64_t device_cus() {
 // rows takes 192 x 160: 1-3 % either way against 256 x 128.)
 // A last, partly filled wave costs 0.7 + 0.3 x its fill of a full one (a half-filled wave
 // measured 0.75-0.98).  Every kernel gives the same bits, so the choice may follow M.
-// (The figures rank the tiles; the 128-row kernel's single waves have since become 10-20 % faster
-// in the same order, and prefill_tile narrows its tiles where smaller ones fit one per CU.)
+// The figures rank the tiles as they were when the table was fitted, and what the kernels have gained
+// since is not the same for all.  One full wave of 256 tiles now, K = 2560, weights from HBM: 256 x
+// 256 / 224 / 192 43.4 39.7 34.7, x 160 / 128 31.1 26.0; 128 x 160 / 128 / 64 20.7 17.3 12.7 (two per CU
+// 33.5 28.5 20.0); 192 x 256 / 160 / 128 35.9 25.5 21.6; 64 x 128 / 64 13.5 9.5 (21.6 14.3).  Under the
+// step before reg_step the single waves of 128 x 64 took 13.6, of 64 x 128 13.7, of 64 x 64 9.6, and two
+// 64 x 64 workgroups a CU 17.0; 128 x 160 and 128 x 128 were the same.  The 96-row and 96-wide forms
+// and 192 x 192 are not in the table: the first two come in through prefill_tile, which narrows a
+// single wave's tile, and so never in place of a 160-wide, 192- or 256-row pick.  Against every
+// forced variant, at 15 row counts from 96 to 4096 of the four projections, the launched tile is the
+// fastest or within the 5 % by which two runs of one kernel differ there, but for qkv at 1024 rows
+// (192 x 160 24.6, 256 x 128 23.7) and at 1300 (128 x 160 31.5, 192 x 192 27.9).
 namespace {
 struct TileVariant {
   int rows, bn;
@@ -877,7 +886,7 @@ double variant_cost(const TileVariant& v, int64_t M, int64_t N, int64_t cus) {
 }
 
 struct PrefillChoice {
-  int rows;  // 64 or 128: tile_gemm_dma; 192 or 256: tile_gemm_256
+  int rows;  // 64, 96 or 128: tile_gemm_dma; 192 or 256: tile_gemm_256
   int bn;
 };
 
