@@ -23,10 +23,12 @@ def _reference(x, w, ws, out_dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("m,n,k", [
-    # 96-row tiles (128-row picks whose 96-row form fits one per CU), rows at their edges.
+    # 96-row tiles (128-row picks whose 96-row form fits one per CU), rows at their edges, and beside
+    # them one size each that a 128x64 (577 rows) and a 64x64 tile (97 rows) takes.
     (512, 2560, 512), (536, 2560, 384), (385, 2500, 640), (577, 2560, 128), (97, 6144, 1024), (1024, 2560, 256),
     (1056, 2560, 896),
-    # 96-wide tiles at every tile height, whose column halves straddle weight-scale blocks.
+    # 96-wide tiles at every tile height, whose column halves straddle weight-scale blocks; one row and
+    # ten columns on, a 96x128 tile.
     (200, 6144, 384), (32, 19456, 256), (63, 19400, 128), (128, 19456, 640), (100, 11008, 512), (864, 2560, 256),
     (865, 2570, 384),
     # K ending inside a group (16 to 112 columns of it), one group and several, every tile height.
